@@ -123,80 +123,77 @@ struct PlanetS {   // planet for the spherical force: mass, radius, angle, softe
 };
 
 // ----------------------------------------------------- reconstruction
-// __logf of a float argument (PEM.cu:13,29): FP32 takes the hardware
-// logarithm; FP64 takes the float logarithm correctly rounded (the double
-// logarithm of the float argument, rounded to float), as the oracle does
-template <typename real> __device__ __forceinline__ real flog(real x);
-template <> __device__ __forceinline__ float flog<float>(float x) { return __logf(x); }
-template <> __device__ __forceinline__ double flog<double>(double x) { return (double)(float)log((double)(float)x); }
+// The power law y^eta of PEM through the logarithm of y (the reference takes
+// __logf of a float argument, PEM.cu:13,29): FP32 takes the hardware base-2
+// logarithm and exponential; FP64 takes the float logarithm correctly
+// rounded (the double logarithm of the float argument, rounded to float), as
+// the oracle does.
+template <typename real> struct Pow;
+template <> struct Pow<float> {
+    static __device__ __forceinline__ float log(float y) { return __builtin_amdgcn_logf(y); }
+    static __device__ __forceinline__ float exp(float z) { return __builtin_amdgcn_exp2f(z); }
+};
+template <> struct Pow<double> {
+    static __device__ __forceinline__ double log(double y) { return (double)(float)::log((double)(float)y); }
+    static __device__ __forceinline__ double exp(double z) { return ::exp(z); }
+};
 
-// Parameters of a cell's sub-cell profile: slopes, mean, and (PEM4) which
-// form each of get_CON_aveL / aveR takes (PEM.cu:51-93), decided once per
-// cell and field since it depends on the slopes only: k = 0 the mean,
-// 1 the parabola, 2 get_PEM_0, 3 get_PEM_1, with exponents eL, eR.
+// Parameters of a cell's sub-cell profile: its mean and slopes (mean less the
+// left edge value, right edge value less the mean).  PEM4 (PEM.cu:51-93) takes
+// the parabola while neither slope exceeds twice the other, the power law of
+// exponent eta = larger / smaller beyond (pl); zl: the right slope is the
+// larger, so that the power law counts from the left edge.  sS: the smaller.
 template <typename real>
 struct Par {
     real sL, a, sR;
-    real eL, eR;
-    int kL, kR;
+    real sS, eta;
+    bool pl, zl;
 };
 
-// the PEM4 branch choices of get_PEM_aveL / aveR (PEM.cu:51-93)
-template <typename real>
-__device__ __forceinline__ void pem_select(Par<real>& p) {
-    if (p.sL * p.sR == real(0)) {
-        p.kL = p.kR = 0;
-        p.eL = p.eR = real(0);
-        return;
+// The profile's mean over the fraction x of the cell next to its left
+// (SIDE -1, get_CON_aveL, recon.cu:424-441) or right (SIDE 1, get_CON_aveR,
+// recon.cu:405-422) edge, less the cell's mean, for N fields at one x.
+// The power law's means (get_PEM_0 / get_PEM_1, PEM.cu:3-48) with eta times
+// the smaller slope put for the larger: the deficit -+D of the mean is
+//   from the edge the power law counts from:  sS (1 - x^eta)
+//   from the other edge:  sS (1 - x) / x (1 - (1 - x)^eta), or below
+//   eta x = 0.001 its series sS eta (1 - v)
+// so the logarithms and the quotient belong to x and are formed once for all
+// fields, and a field costs one exponential and a handful of products: with
+// 1e-4 noise on the density some lane of nearly every wave takes the power law
+// in some field, and the forms evaluated field by field, each behind its own
+// branches with a logarithm and a division, kept 40-52 % of the lanes idle in
+// the radial and azimuthal sweeps, which issue instructions on every cycle
+// (384x1536x64 step 4.69 -> 4.17 ms, 96x384x64 333 -> 285 us).
+template <int RECON, int SIDE, int N, typename real>
+__device__ __forceinline__ void edge_means(real x, const Par<real>* const (&P)[N], real (&dev)[N]) {
+    bool any = false;
+#pragma unroll
+    for (int f = 0; f < N; ++f) {
+        const real l = P[f]->sL, r = P[f]->sR;
+        dev[f] = SIDE < 0 ? fma(x, fma(-x, l - r, real(2) * l - r), -l) : fma(x, fma(-x, l - r, l - real(2) * r), r);
+        any = any || P[f]->pl;
     }
-    const real rr = FM<real>::div(p.sR, p.sL), rl = FM<real>::div(p.sL, p.sR);
-    p.kL = rr >= real(1) ? (rr <= real(2) ? 1 : 2) : (rl <= real(2) ? 1 : 3);
-    p.eL = rr >= real(1) ? rr : rl;
-    p.kR = rr > real(1) ? (rr <= real(2) ? 1 : 3) : (rl <= real(2) ? 1 : 2);
-    p.eR = rr > real(1) ? rr : rl;
-}
-
-// get_PEM_0 / get_PEM_1 (PEM.cu:3-48) through one logarithm and one
-// exponential: with y = x (PEM_0) or 1 - x (PEM_1), E = y^eta; PEM_0 is E,
-// PEM_1 is (1 - x)(E - 1)/(eta x) + 1 or its series below eta x = 0.001 (so
-// lanes of a wave that take different forms share the transcendental work).
-// get_PEM_1's x >= 1 assignment is overwritten by the branch after it
-// (PEM.cu:23-27) and has no counterpart.
-template <typename real>
-__device__ __forceinline__ real pem01(bool zero_form, real x, real S, real aB, real eta) {
-    const real y = zero_form ? x : real(1) - x;
-    const real E = y == real(0) ? real(0) : FM<real>::exp(eta * flog(y));
-    real v;
-    if (zero_form) {
-        v = E;
-    } else if (eta * x > real(0.001)) {
-        v = FM<real>::div(y * (E - real(1)), eta * x) + real(1);
-    } else {
-        real t = (eta + real(1)) * x / real(2);
-        v = t;
-        t *= -(eta - real(1)) * x / real(3);
-        v += t;
-        t *= -(eta - real(2)) * x / real(4);
-        v += t;
-        t *= -(eta - real(3)) * x / real(5);
-        v += t;
+    if (RECON == 6 || !any) return;
+    const real y = real(1) - x;
+    const real lx = Pow<real>::log(x), ly = Pow<real>::log(y);
+    const real yx = FM<real>::div(y, x);
+#pragma unroll
+    for (int f = 0; f < N; ++f) {
+        const bool z = (SIDE < 0) == P[f]->zl;
+        const real eta = P[f]->eta;
+        real D = P[f]->sS * (z ? real(1) : yx) * (real(1) - Pow<real>::exp(eta * (z ? lx : ly)));
+        const real ex = eta * x;
+        if (P[f]->pl && !z && !(ex > real(0.001))) {
+            // the terms beyond the third are below FP32's last place here
+            real v = sizeof(real) == 8 ? real(1) - (eta - real(3)) * x * real(0.2) : real(1);
+            v = real(1) - (eta - real(2)) * x * real(0.25) * v;
+            v = real(1) - (eta - real(1)) * x * real(1.0 / 3.0) * v;
+            v = (eta + real(1)) * x * real(0.5) * v;
+            D = P[f]->sS * eta * (real(1) - v);
+        }
+        dev[f] = P[f]->pl ? (SIDE < 0 ? -D : D) : dev[f];
     }
-    return aB + S * v;
-}
-
-// get_CON_aveL (recon.cu:424-441): mean over the first fraction q
-template <int RECON, typename real>
-__device__ __forceinline__ real avgL(real q, const Par<real>& p) {
-    if (RECON == 6 || p.kL == 1) return aveL(q, p.sL, p.a, p.sR);
-    if (p.kL == 0) return p.a;
-    return pem01(p.kL == 2, q, p.sL, p.a - p.sL, p.eL);
-}
-// get_CON_aveR (recon.cu:405-422): mean over the cell from q to its right edge
-template <int RECON, typename real>
-__device__ __forceinline__ real avgR(real q, const Par<real>& p) {
-    if (RECON == 6 || p.kR == 1) return aveR(real(1) - q, p.sL, p.a, p.sR);
-    if (p.kR == 0) return p.a;
-    return pem01(p.kR == 2, real(1) - q, -p.sR, p.a + p.sR, p.eR);
 }
 
 // 4th-order limited slopes (recon.cu:216-378); under RECON 6 also the
@@ -205,10 +202,10 @@ template <int RECON, typename real>
 __device__ __forceinline__ Par<real> params(real am2, real am1, real a0, real ap1, real ap2, const real* w, real flat) {
     Par<real> p;
     p.a = a0;
+    p.sS = p.eta = real(0);
+    p.pl = p.zl = false;
     if (RECON == 6) {
         slopes(am2, am1, a0, ap1, ap2, w[0], w[1], w[2], w[3], w[4], w[5], flat, p.sL, p.sR);
-        p.kL = p.kR = 1;
-        p.eL = p.eR = real(0);
         return p;
     }
     real d0 = am1 - am2, d1 = a0 - am1, d2 = ap1 - a0, d3 = ap2 - ap1;
@@ -216,95 +213,62 @@ __device__ __forceinline__ Par<real> params(real am2, real am1, real a0, real ap
     real r = w[3] * d1 + w[4] * d2 + w[5] * d3;
     l = copysign(fmin(fabs(l), fabs(d1)), d1);
     r = copysign(fmin(fabs(r), fabs(d2)), d2);
-    if (r * l <= real(0)) {
+    if (r * l <= real(0)) {   // also where one of them is zero: the profile is its mean
         l = real(0);
         r = real(0);
     }
     p.sL = l;
     p.sR = r;
-    pem_select(p);
-    return p;
-}
-// the same parameters about a zero mean: avgL / avgR of them is the sub-cell
-// mean less the cell's own (both are affine in the mean with unit weight)
-template <typename real>
-__device__ __forceinline__ Par<real> zero_mean(Par<real> p) {
-    p.a = real(0);
+    const real al = fabs(l), ar = fabs(r);
+    p.zl = ar > al;
+    p.pl = fmax(al, ar) > real(2) * fmin(al, ar);
+    p.sS = p.zl ? l : r;
+    p.eta = FM<real>::div(p.zl ? r : l, p.sS);   // used where pl: there the smaller is not zero
     return p;
 }
 
-// set_state (states.cu:1-135) for an adiabatic gas: the state right of the
-// cell's left edge (from the cell's means over its first fractions, R side)
-// and left of its right edge (L side).  P: parameters of rho, p, u, v, w;
-// rc, pc, uc: the cell's values; dts: the sweep's time step over its length
-// unit (dt / rad); idx = 1 / width.
+// set_state (states.cu:1-135) for an adiabatic gas: the half-step state at
+// the left edge of a cell (SIDE -1, the R state of that interface) or at its
+// right edge (SIDE 1, the L state).  P: parameters of rho, p, u, v, w; rc,
+// pc, uc, cs: the cell's values and sound speed; dts: the sweep's time step
+// over its length unit (dt / rad); idx = 1 / width.
 // The traced pressure S[1] is returned as its deviation from the edge's
 // reference pressure pref (the mean of the two cells' pressures), given the
 // cell's own deviation pdev = p - pref: the pressure's sub-cell means enter
 // as their differences from the cell's pressure, so the pressure
 // differences of the update are formed from numbers of their own size.
 // S[1] is p0 exp_lim(gam u_) - pref = (p0 - pref) + p0 (exp_lim(gam u_) - 1).
+// One reciprocal square root y = 1 / sqrt(gam p0 r0) gives the traced sound
+// speed gam p0 y, its reciprocal r0 y and 1 / (r0 cs) = y.
 template <typename real>
 __device__ __forceinline__ real exp_lim_m1(real x) {   // exp_lim(x) - 1
     return fmax(x, real(1.0e-6) - real(1));
 }
-template <int RECON, typename real>
-__device__ __forceinline__ void trace_R(const Par<real>* P, real rc, real pc, real uc, real pdev, real gam, real dts,
-                                        real idx, real* S) {
-    const real hdt = real(0.5) * dts;
-    real cs = FM<real>::sqrt(FM<real>::div(gam * pc, rc));
-    real q = lim01((cs - fmin(uc, real(0))) * dts * idx);
+template <int RECON, int SIDE, typename real>
+__device__ __forceinline__ void trace(const Par<real>* P, real rc, real pc, real uc, real pdev, real cs, real gam,
+                                      real dts, real idx, real* S) {
+    const real sg = real(SIDE), dti = dts * idx;
+    real d1[1];
+    edge_means<RECON, SIDE, 1, real>(lim01((fmax(sg * uc, real(0)) + cs) * dti), {&P[2]}, d1);
+    const real w = fmax(sg * (uc + d1[0]), real(0));   // the edge's own speed toward it
+    real m0[3];
+    edge_means<RECON, SIDE, 3, real>(lim01(w * dti), {&P[0], &P[1], &P[2]}, m0);
     const real rmin = rc * real(1.0e-10), pmin = pc * real(1.0e-10);
-    const real ur = avgL<RECON>(q, P[2]);
-    const real dis = fmin(ur, real(0)) * dts;
-    q = lim01(-dis * idx);
-    const Par<real> Pz = zero_mean(P[1]);
-    const real dp0 = avgL<RECON>(q, Pz);
-    real r0 = avgL<RECON>(q, P[0]), p0 = pc + dp0, u0 = avgL<RECON>(q, P[2]);
-    r0 = fmax(r0, rmin);
-    const bool pfl = p0 < pmin;
-    p0 = fmax(p0, pmin);
-    cs = FM<real>::sqrt(FM<real>::div(gam * p0, r0));
-    q = lim01((cs * dts - dis) * idx);
-    const real dp_ = avgL<RECON>(q, Pz);
-    real u_ = avgL<RECON>(q, P[2]);
-    const real f = FM<real>::div(real(2), cs * dts) * (-hdt);
-    u_ = (u_ - u0) * f;
-    const real p_ = (pfl ? (pc + dp_) - p0 : dp_ - dp0) * f;
+    const real r0 = fmax(rc + m0[0], rmin), u0 = uc + m0[2];
+    real dp0 = m0[1], p0 = pc + dp0;
+    if (p0 < pmin) {
+        p0 = pmin;
+        dp0 = pmin - pc;
+    }
+    const real gp = gam * p0, y = FM<real>::rsqrt(gp * r0);
+    real m1[4];
+    edge_means<RECON, SIDE, 4, real>(lim01((w + gp * y) * dti), {&P[1], &P[2], &P[3], &P[4]}, m1);
+    const real u_ = sg * ((uc + m1[1]) - u0) * (r0 * y);
     S[0] = r0 * exp_lim(u_);
-    S[1] = (pfl ? p0 - (pc - pdev) : pdev + dp0) + p0 * exp_lim_m1(gam * u_);
-    S[2] = u0 + FM<real>::div(p_, r0);
-    S[3] = avgL<RECON>(q, P[3]);
-    S[4] = avgL<RECON>(q, P[4]);
-}
-template <int RECON, typename real>
-__device__ __forceinline__ void trace_L(const Par<real>* P, real rc, real pc, real uc, real pdev, real gam, real dts,
-                                        real idx, real* S) {
-    const real hdt = real(0.5) * dts;
-    real cs = FM<real>::sqrt(FM<real>::div(gam * pc, rc));
-    real q = lim01(real(1) - (fmax(uc, real(0)) + cs) * dts * idx);
-    const real rmin = rc * real(1.0e-10), pmin = pc * real(1.0e-10);
-    const real ul = avgR<RECON>(q, P[2]);
-    const real dis = fmax(ul, real(0)) * dts;
-    q = lim01(real(1) - dis * idx);
-    const Par<real> Pz = zero_mean(P[1]);
-    const real dp0 = avgR<RECON>(q, Pz);
-    real r0 = avgR<RECON>(q, P[0]), p0 = pc + dp0, u0 = avgR<RECON>(q, P[2]);
-    r0 = fmax(r0, rmin);
-    const bool pfl = p0 < pmin;
-    p0 = fmax(p0, pmin);
-    cs = FM<real>::sqrt(FM<real>::div(gam * p0, r0));
-    q = lim01(real(1) - (dis + cs * dts) * idx);
-    const real dp_ = avgR<RECON>(q, Pz);
-    real u_ = avgR<RECON>(q, P[2]);
-    const real f = FM<real>::div(real(2), cs * dts) * (-hdt);
-    u_ = (u0 - u_) * f;
-    const real p_ = (pfl ? p0 - (pc + dp_) : dp0 - dp_) * f;
-    S[0] = r0 * exp_lim(u_);
-    S[1] = (pfl ? p0 - (pc - pdev) : pdev + dp0) + p0 * exp_lim_m1(gam * u_);
-    S[2] = u0 + FM<real>::div(p_, r0);
-    S[3] = avgR<RECON>(q, P[3]);
-    S[4] = avgR<RECON>(q, P[4]);
+    S[1] = (pdev + dp0) + p0 * exp_lim_m1(gam * u_);
+    S[2] = u0 + sg * (m1[0] - dp0) * y;
+    S[3] = P[3].a + m1[2];
+    S[4] = P[4].a + m1[3];
 }
 
 // wave_speeds (wave_speeds.cu:24-35,288-333) and HLLC_fluxes (HLLC.cu:2-77)
@@ -533,8 +497,8 @@ __global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<re
         for (int m = 0; m < 6; ++m) wl[m] = DIR == 1 ? w[m] : w[(size_t)m * ws];
         const real* q = raw + e;
         real flat = real(0);
+        const real cs = FM<real>::sqrt(FM<real>::div(a.gam * q[RS], q[0]));
         if (RECON == 6) {
-            const real cs = FM<real>::sqrt(FM<real>::div(a.gam * q[RS], q[0]));
             const real* pp = q + RS;
             const real* uu = q + 2 * RS;
             flat = flatten5(pp[-2 * R], pp[-R], pp[0], pp[R], pp[2 * R], uu[-R], uu[0], uu[R], cs);
@@ -550,8 +514,8 @@ __global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<re
         // precision, so these carry no rounding of the pressure itself
         const real pdl = real(0.5) * (q[RS] - q[RS - R]), pdr = real(0.5) * (q[RS] - q[RS + R]);
         real SR[NF], SL[NF];
-        trace_R<RECON>(P, q[0], q[RS], q[2 * RS], pdl, a.gam, dts, idx, SR);
-        trace_L<RECON>(P, q[0], q[RS], q[2 * RS], pdr, a.gam, dts, idx, SL);
+        trace<RECON, -1>(P, q[0], q[RS], q[2 * RS], pdl, cs, a.gam, dts, idx, SR);
+        trace<RECON, 1>(P, q[0], q[RS], q[2 * RS], pdr, cs, a.gam, dts, idx, SL);
         for (int f = 0; f < NF; ++f) {
             TRs[f * RS + e] = SR[f];
             TLs[f * RS + e] = SL[f];
@@ -709,14 +673,24 @@ __global__ __launch_bounds__(SPH_BT) void k3_orbadv(SphK<real> a, double dt, int
         const real dte = FM<real>::div((real)dt, a.xc[i + NPAD] * a.sinz[k0 + NPAD]);
         const bool up = speed > real(0);
         const int cs = up ? s - 1 : s;
-        const real q = up ? lim01(real(1) - speed * dte * a.idy) : lim01(-speed * dte * a.idy);
+        const real q = lim01(fabs(speed) * dte * a.idy);
         const real* x = raw + cs * R + r;
+        // the upwind cell's mean next to this interface: its right edge, or
+        // its left one; the first is the second of the mirrored profile,
+        // whose slopes are -sR and -sL
+        Par<real> P[NF];
         real D[NF];
         for (int f = 0; f < NF; ++f) {
             const real* y = x + f * RS;
-            const Par<real> P = params<RECON>(y[-2 * R], y[-R], y[0], y[R], y[2 * R], a.yw, real(0));
-            D[f] = up ? avgR<RECON>(q, P) : avgL<RECON>(q, P);
+            P[f] = params<RECON>(y[-2 * R], y[-R], y[0], y[R], y[2 * R], a.yw, real(0));
+            const real l = P[f].sL;
+            P[f].sL = up ? -P[f].sR : l;
+            P[f].sR = up ? -l : P[f].sR;
+            P[f].sS = up ? -P[f].sS : P[f].sS;
+            P[f].zl = P[f].zl != up;
         }
+        edge_means<RECON, -1, NF, real>(q, {&P[0], &P[1], &P[2], &P[3], &P[4]}, D);
+        for (int f = 0; f < NF; ++f) D[f] += P[f].a;
         FX[e] = D[0] * speed;
         FX[RS + e] = D[1] * speed;
         for (int f = 2; f < NF; ++f) FX[f * RS + e] = D[f] * D[0] * speed;
