@@ -20,10 +20,10 @@
 // (boundary type 2).
 //
 // Sweeps stage a tile of R rows x S cells (S = segment + 6 ghost or halo
-// cells) in LDS; thread t owns elements e = t, t + 256, ... with e = s*R + r,
-// so consecutive threads hold consecutive radii of the strided sweeps (the
-// coalesced direction of the global loads) and the row neighbours of an
-// element sit R apart in LDS.  Phases: load -> per cell: reconstruction and
+// cells) in LDS; thread t owns elements e = t, t + 512, ... with e = s*R + r
+// in the strided sweeps, so that consecutive threads hold consecutive radii
+// (the coalesced direction of the global loads) and the row neighbours of an
+// element sit R apart in LDS, and e = r*S + s in the radial one.  Phases: load -> per cell: reconstruction and
 // the two characteristic-traced states -> per interface: HLLC -> per cell:
 // flux and pressure-source differences, the conservative update.
 
@@ -49,14 +49,12 @@ namespace pg {
 namespace {
 
 constexpr int NF = 5;            // rho, p, u, vp, w
-constexpr int SPH_BT = 256;      // threads per block of the pointwise kernels and the radial sweep
-constexpr int SPH_BT2 = 512;     // threads per block of the strided sweeps (about one element each)
-constexpr int SPH_BTX = 256;     // most threads per radial-sweep block (one per LDS slot)
+constexpr int SPH_BT = 256;      // threads per block of the pointwise kernels
+constexpr int SPH_BT2 = 512;     // threads per block of the sweeps (about one element each)
 constexpr int SPH_R = 8;         // rows per strided-sweep block
 // azimuthal segment per block: with its 6 halo rows, 8 radii x 64 slots fill
 // a 512-thread block (and two passes of a 256-thread one) exactly (64 rows:
-// 560 slots, a partly filled extra pass; 1091 -> 1050 us for the azimuthal
-// sweep, 591 -> 555 us for the orbital advection of the 384x1536x64 disk)
+// 560 slots, a partly filled extra pass, 4-6 % slower)
 constexpr int SPH_TY = 58;
 constexpr int SPH_ZMAX = 100;    // polar cells: the whole column is one tile (FP64: 102 KB of LDS)
 
@@ -101,21 +99,43 @@ struct SphK {
     real dy, idy;
     double dy_d;
     real gam;
-    int tx;   // radial segment of the radial sweep (sph_tx)
+    int tx, xr;   // radial sweep: cells of a segment, rows of a block (radial_tile)
+    int xm;       // (1 << 20) / (tx + 2 NPAD) + 1: t / (tx + 2 NPAD) = (t * xm) >> 20 for t < SPH_BT2
 };
 
-// Radial segment of the radial sweep: the row cut into the fewest equal
-// parts whose slots (segment + 2 NPAD) fit one block of SPH_BTX threads, so
-// every thread holds one slot and no block runs half empty (a 384-radius row
-// is two 198-slot blocks of 256 threads: a CU holds more of them than of one
-// 390-slot block of 448 threads, and one block's loads hide behind the
-// others' arithmetic: 1343 -> 1219 us on the 384x1536x64 disk; 128-thread
-// blocks of 102 slots 1240-1256 us).
-inline int sph_tx(int nx) {
-    const int parts = (nx + SPH_BTX - 2 * NPAD - 1) / (SPH_BTX - 2 * NPAD);
-    return (nx + parts - 1) / parts;
+// Tile of the radial sweep: xr rows x a segment of tx cells.  The row is cut
+// into equal segments, and as many rows as fit SPH_BT2 threads (one per slot,
+// segment + 2 NPAD slots a row; half as many in FP64, whose PEM4 sweep needs
+// 160 VGPRs: 84 us against 127 on a 96x192x32 disk) make a block; of all cuts
+// the one that puts the most cells into a block's threads, so that few lanes issue instructions
+// for halo cells or for nothing (a 384-radius row: five rows of four 102-slot
+// segments fill 480 of 512 lanes with cells, one row's two 198-slot segments
+// 192 of 256: radial sweep of the 384x1536x64 disk 1210 -> 1140 us, its lanes
+// in use 75 -> 88 %).  A small disk takes fewer rows, down to one, so that the
+// blocks still cover the chip's 256 CUs eight times (a 101x190x33 disk is 1 %
+// slower with four rows in 1568 blocks than with three in 2090).
+struct RadialTile {
+    int tx, xr;
+};
+inline RadialTile radial_tile(int nx, long rows, int es) {
+    const int most_threads = es == 8 ? SPH_BT2 / 2 : SPH_BT2;
+    RadialTile best{0, 0};
+    double most = 0.0;
+    for (int parts = (nx + most_threads - 2 * NPAD - 1) / (most_threads - 2 * NPAD); parts <= nx; ++parts) {
+        const int tx = (nx + parts - 1) / parts;
+        if (best.tx && tx < 32) break;   // the halo alone is 16 % there
+        const long nseg = (nx + tx - 1) / tx;
+        int xr = most_threads / (tx + 2 * NPAD);
+        while (xr > 1 && nseg * ((rows + xr - 1) / xr) < 2048) --xr;
+        const int threads = (xr * (tx + 2 * NPAD) + 63) / 64 * 64;
+        const double use = (double)nx * xr / ((double)nseg * threads);
+        if (use > most) {
+            most = use;
+            best = RadialTile{tx, xr};
+        }
+    }
+    return best;
 }
-inline int sph_bx(int nx) { return (sph_tx(nx) + 2 * NPAD + 63) / 64 * 64; }
 
 template <typename real>
 struct PlanetS {   // planet for the spherical force: mass, radius, angle, softening
@@ -123,76 +143,78 @@ struct PlanetS {   // planet for the spherical force: mass, radius, angle, softe
 };
 
 // ----------------------------------------------------- reconstruction
-// The power law y^eta of PEM through the logarithm of y (the reference takes
-// __logf of a float argument, PEM.cu:13,29): FP32 takes the hardware base-2
-// logarithm and exponential; FP64 takes the float logarithm correctly
-// rounded (the double logarithm of the float argument, rounded to float), as
-// the oracle does.
-template <typename real> struct Pow;
-template <> struct Pow<float> {
-    static __device__ __forceinline__ float log(float y) { return __builtin_amdgcn_logf(y); }
-    static __device__ __forceinline__ float exp(float z) { return __builtin_amdgcn_exp2f(z); }
-};
-template <> struct Pow<double> {
-    static __device__ __forceinline__ double log(double y) { return (double)(float)::log((double)(float)y); }
-    static __device__ __forceinline__ double exp(double z) { return ::exp(z); }
-};
+// The natural logarithm of a fraction in [0, 1] (__logf of a float argument,
+// PEM.cu:13,29) and the exponential of a multiple of it.  FP32: the hardware
+// base-2 logarithm times ln 2 in two parts, as __logf forms it, without its
+// scaling of denormal arguments (their powers here, above the second, are zero
+// either way) and with a finite number for the logarithm of zero, which every
+// power also takes to zero.  FP64 takes the float logarithm correctly rounded
+// (the double logarithm of the float argument, rounded to float), as the
+// oracle does.
+template <typename real> __device__ __forceinline__ real flog(real x);
+template <> __device__ __forceinline__ float flog<float>(float x) {
+    const float r = fmaxf(__builtin_amdgcn_logf(x), -1024.0f), ln2 = 0x1.62e42ep-1f, ln2_lo = 0x1.efa39ep-25f;
+    const float h = r * ln2;
+    return fmaf(r, ln2, fmaf(r, ln2_lo, fmaf(r, ln2, -h)));
+}
+template <> __device__ __forceinline__ double flog<double>(double x) { return (double)(float)log((double)(float)x); }
 
 // Parameters of a cell's sub-cell profile: its mean and slopes (mean less the
 // left edge value, right edge value less the mean).  PEM4 (PEM.cu:51-93) takes
-// the parabola while neither slope exceeds twice the other, the power law of
+// the parabola while neither slope exceeds twice the other, a power law of
 // exponent eta = larger / smaller beyond (pl); zl: the right slope is the
-// larger, so that the power law counts from the left edge.  sS: the smaller.
+// larger, so that the power law counts from the left edge.
 template <typename real>
 struct Par {
     real sL, a, sR;
-    real sS, eta;
+    real eta;
     bool pl, zl;
 };
 
 // The profile's mean over the fraction x of the cell next to its left
-// (SIDE -1, get_CON_aveL, recon.cu:424-441) or right (SIDE 1, get_CON_aveR,
-// recon.cu:405-422) edge, less the cell's mean, for N fields at one x.
-// The power law's means (get_PEM_0 / get_PEM_1, PEM.cu:3-48) with eta times
-// the smaller slope put for the larger: the deficit -+D of the mean is
-//   from the edge the power law counts from:  sS (1 - x^eta)
-//   from the other edge:  sS (1 - x) / x (1 - (1 - x)^eta), or below
-//   eta x = 0.001 its series sS eta (1 - v)
-// so the logarithms and the quotient belong to x and are formed once for all
-// fields, and a field costs one exponential and a handful of products: with
-// 1e-4 noise on the density some lane of nearly every wave takes the power law
-// in some field, and the forms evaluated field by field, each behind its own
-// branches with a logarithm and a division, kept 40-52 % of the lanes idle in
-// the radial and azimuthal sweeps, which issue instructions on every cycle
-// (384x1536x64 step 4.69 -> 4.17 ms, 96x384x64 333 -> 285 us).
+// (SIDE -1, get_CON_aveL, recon.cu:424-441) or right edge (SIDE 1,
+// get_CON_aveR, recon.cu:405-422), for N fields at one x.  The power law's
+// means (get_PEM_0 / get_PEM_1, PEM.cu:3-48) take one logarithm and one
+// exponential: with y = x counting from the law's own edge or y = 1 - x from
+// the other, E = y^eta, the mean is E or (1 - x)(E - 1)/(eta x) + 1, below
+// eta x = 0.001 its series.  (get_PEM_1's x >= 1 assignment is overwritten by
+// the branch after it, PEM.cu:23-27, and has no counterpart.)
+// The logarithms belong to x and are formed once for all fields, under one
+// branch: with 1e-4 noise on the density some lane of nearly every wave takes
+// the power law in some field, and the forms evaluated field by field, each
+// behind its own branches, kept 40-52 % of the lanes idle in the radial and
+// azimuthal sweeps, which issue instructions on every cycle (384x1536x64 step
+// 4.69 -> 4.14 ms, 96x384x64 332 -> 292 us with the radial sweep's tiles).
 template <int RECON, int SIDE, int N, typename real>
-__device__ __forceinline__ void edge_means(real x, const Par<real>* const (&P)[N], real (&dev)[N]) {
+__device__ __forceinline__ void edge_means(real x, const Par<real> (&P)[N], real (&m)[N]) {
     bool any = false;
 #pragma unroll
     for (int f = 0; f < N; ++f) {
-        const real l = P[f]->sL, r = P[f]->sR;
-        dev[f] = SIDE < 0 ? fma(x, fma(-x, l - r, real(2) * l - r), -l) : fma(x, fma(-x, l - r, l - real(2) * r), r);
-        any = any || P[f]->pl;
+        m[f] = SIDE < 0 ? aveL(x, P[f].sL, P[f].a, P[f].sR) : aveR(x, P[f].sL, P[f].a, P[f].sR);
+        any = any || P[f].pl;
     }
     if (RECON == 6 || !any) return;
     const real y = real(1) - x;
-    const real lx = Pow<real>::log(x), ly = Pow<real>::log(y);
-    const real yx = FM<real>::div(y, x);
+    const real lx = flog(x), ly = flog(y);
 #pragma unroll
     for (int f = 0; f < N; ++f) {
-        const bool z = (SIDE < 0) == P[f]->zl;
-        const real eta = P[f]->eta;
-        real D = P[f]->sS * (z ? real(1) : yx) * (real(1) - Pow<real>::exp(eta * (z ? lx : ly)));
+        const bool z = (SIDE < 0) == P[f].zl;
+        const real eta = P[f].eta;
+        const real S = SIDE < 0 ? P[f].sL : -P[f].sR;   // mean less the edge's value, as the edge sees it
+        const real E = FM<real>::exp(eta * (z ? lx : ly));
         const real ex = eta * x;
-        if (P[f]->pl && !z && !(ex > real(0.001))) {
-            // the terms beyond the third are below FP32's last place here
-            real v = sizeof(real) == 8 ? real(1) - (eta - real(3)) * x * real(0.2) : real(1);
-            v = real(1) - (eta - real(2)) * x * real(0.25) * v;
-            v = real(1) - (eta - real(1)) * x * real(1.0 / 3.0) * v;
-            v = (eta + real(1)) * x * real(0.5) * v;
-            D = P[f]->sS * eta * (real(1) - v);
+        real v = z ? E : FM<real>::div(y * (E - real(1)), ex) + real(1);
+        if (P[f].pl && !z && !(ex > real(0.001))) {
+            real t = (eta + real(1)) * x * real(0.5);
+            v = t;
+            t *= -(eta - real(1)) * x * real(1.0 / 3.0);
+            v += t;
+            t *= -(eta - real(2)) * x * real(0.25);
+            v += t;
+            t *= -(eta - real(3)) * x * real(0.2);
+            v += t;
         }
-        dev[f] = P[f]->pl ? (SIDE < 0 ? -D : D) : dev[f];
+        m[f] = P[f].pl ? (P[f].a - S) + S * v : m[f];
     }
 }
 
@@ -202,7 +224,7 @@ template <int RECON, typename real>
 __device__ __forceinline__ Par<real> params(real am2, real am1, real a0, real ap1, real ap2, const real* w, real flat) {
     Par<real> p;
     p.a = a0;
-    p.sS = p.eta = real(0);
+    p.eta = real(0);
     p.pl = p.zl = false;
     if (RECON == 6) {
         slopes(am2, am1, a0, ap1, ap2, w[0], w[1], w[2], w[3], w[4], w[5], flat, p.sL, p.sR);
@@ -219,18 +241,24 @@ __device__ __forceinline__ Par<real> params(real am2, real am1, real a0, real ap
     }
     p.sL = l;
     p.sR = r;
-    const real al = fabs(l), ar = fabs(r);
-    p.zl = ar > al;
-    p.pl = fmax(al, ar) > real(2) * fmin(al, ar);
-    p.sS = p.zl ? l : r;
-    p.eta = FM<real>::div(p.zl ? r : l, p.sS);   // used where pl: there the smaller is not zero
+    p.zl = fabs(r) > fabs(l);
+    p.eta = FM<real>::div(p.zl ? r : l, p.zl ? l : r);
+    p.pl = p.eta > real(2);   // false where both are zero
+    return p;
+}
+
+// the same parameters about a zero mean: their edge means are the sub-cell
+// mean less the cell's own (affine in the mean with unit weight)
+template <typename real>
+__device__ __forceinline__ Par<real> zero_mean(Par<real> p) {
+    p.a = real(0);
     return p;
 }
 
 // set_state (states.cu:1-135) for an adiabatic gas: the half-step state at
 // the left edge of a cell (SIDE -1, the R state of that interface) or at its
 // right edge (SIDE 1, the L state).  P: parameters of rho, p, u, v, w; rc,
-// pc, uc, cs: the cell's values and sound speed; dts: the sweep's time step
+// pc, uc: the cell's values, cs its sound speed; dts: the sweep's time step
 // over its length unit (dt / rad); idx = 1 / width.
 // The traced pressure S[1] is returned as its deviation from the edge's
 // reference pressure pref (the mean of the two cells' pressures), given the
@@ -238,37 +266,43 @@ __device__ __forceinline__ Par<real> params(real am2, real am1, real a0, real ap
 // as their differences from the cell's pressure, so the pressure
 // differences of the update are formed from numbers of their own size.
 // S[1] is p0 exp_lim(gam u_) - pref = (p0 - pref) + p0 (exp_lim(gam u_) - 1).
-// One reciprocal square root y = 1 / sqrt(gam p0 r0) gives the traced sound
-// speed gam p0 y, its reciprocal r0 y and 1 / (r0 cs) = y.
 template <typename real>
 __device__ __forceinline__ real exp_lim_m1(real x) {   // exp_lim(x) - 1
     return fmax(x, real(1.0e-6) - real(1));
 }
+// the fraction next to the edge that a distance of X cell widths covers (the
+// right edge's counted from the left, as the reference does)
+template <int SIDE, typename real>
+__device__ __forceinline__ real edge_fraction(real X) {
+    return SIDE < 0 ? lim01(X) : real(1) - lim01(real(1) - X);
+}
 template <int RECON, int SIDE, typename real>
 __device__ __forceinline__ void trace(const Par<real>* P, real rc, real pc, real uc, real pdev, real cs, real gam,
                                       real dts, real idx, real* S) {
-    const real sg = real(SIDE), dti = dts * idx;
-    real d1[1];
-    edge_means<RECON, SIDE, 1, real>(lim01((fmax(sg * uc, real(0)) + cs) * dti), {&P[2]}, d1);
-    const real w = fmax(sg * (uc + d1[0]), real(0));   // the edge's own speed toward it
-    real m0[3];
-    edge_means<RECON, SIDE, 3, real>(lim01(w * dti), {&P[0], &P[1], &P[2]}, m0);
+    const real hdt = real(0.5) * dts;
     const real rmin = rc * real(1.0e-10), pmin = pc * real(1.0e-10);
-    const real r0 = fmax(rc + m0[0], rmin), u0 = uc + m0[2];
-    real dp0 = m0[1], p0 = pc + dp0;
-    if (p0 < pmin) {
-        p0 = pmin;
-        dp0 = pmin - pc;
-    }
-    const real gp = gam * p0, y = FM<real>::rsqrt(gp * r0);
-    real m1[4];
-    edge_means<RECON, SIDE, 4, real>(lim01((w + gp * y) * dti), {&P[1], &P[2], &P[3], &P[4]}, m1);
-    const real u_ = sg * ((uc + m1[1]) - u0) * (r0 * y);
+    const Par<real> Pz = zero_mean(P[1]);
+    real m1[1], m3[3], m4[4];
+    const Par<real> P1[1] = {P[2]}, P3[3] = {P[0], Pz, P[2]}, P4[4] = {Pz, P[2], P[3], P[4]};
+    edge_means<RECON, SIDE, 1>(edge_fraction<SIDE>((SIDE < 0 ? cs - fmin(uc, real(0)) : fmax(uc, real(0)) + cs) * dts * idx),
+                               P1, m1);
+    const real dis = (SIDE < 0 ? fmin(m1[0], real(0)) : fmax(m1[0], real(0))) * dts;   // toward the edge
+    edge_means<RECON, SIDE, 3>(edge_fraction<SIDE>(SIDE < 0 ? -dis * idx : dis * idx), P3, m3);
+    const real r0 = fmax(m3[0], rmin), dp0 = m3[1], u0 = m3[2];
+    real p0 = pc + dp0;
+    const bool pfl = p0 < pmin;
+    p0 = fmax(p0, pmin);
+    cs = FM<real>::sqrt(FM<real>::div(gam * p0, r0));
+    edge_means<RECON, SIDE, 4>(edge_fraction<SIDE>((SIDE < 0 ? cs * dts - dis : dis + cs * dts) * idx), P4, m4);
+    const real dp_ = m4[0];
+    const real f = FM<real>::div(real(2), cs * dts) * (-hdt);
+    const real u_ = (SIDE < 0 ? m4[1] - u0 : u0 - m4[1]) * f;
+    const real p_ = SIDE < 0 ? (pfl ? (pc + dp_) - p0 : dp_ - dp0) * f : (pfl ? p0 - (pc + dp_) : dp0 - dp_) * f;
     S[0] = r0 * exp_lim(u_);
-    S[1] = (pdev + dp0) + p0 * exp_lim_m1(gam * u_);
-    S[2] = u0 + sg * (m1[0] - dp0) * y;
-    S[3] = P[3].a + m1[2];
-    S[4] = P[4].a + m1[3];
+    S[1] = (pfl ? p0 - (pc - pdev) : pdev + dp0) + p0 * exp_lim_m1(gam * u_);
+    S[2] = u0 + FM<real>::div(p_, r0);
+    S[3] = m4[2];
+    S[4] = m4[3];
 }
 
 // wave_speeds (wave_speeds.cu:24-35,288-333) and HLLC_fluxes (HLLC.cu:2-77)
@@ -315,10 +349,10 @@ __device__ __forceinline__ void hllc_adi(const real* L, const real* R, real pref
 }
 
 // update_Cell (sweeps.cu:218-261), EOS_flag 2, internal_e_flag 1, on the
-// stored fields (rho, p, u, vp, w); D: changes of mass, internal energy and
-// the momenta of u, vp, w
+// stored fields (rho, p, u, vp, w); D: changes of mass, internal energy (over
+// fac) and the momenta of u, vp, w
 template <typename real>
-__device__ __forceinline__ void update_cell(real* c, const real* D, real gam) {
+__device__ __forceinline__ void update_cell(real* c, const real* D, real fac, real gam) {
     const real rmin = fmax(c[0] * real(1.0e-10), real(1.0e-10));
     const real pmin = fmax(c[1] * real(1.0e-10), real(1.0e-10));
     const real E = FM<real>::div(c[1], (gam - real(1)) * c[0]) * c[0];
@@ -334,7 +368,7 @@ __device__ __forceinline__ void update_cell(real* c, const real* D, real gam) {
     c[2] += (D[2] - c[2] * D[0]) * ir;
     c[3] += (D[3] - c[3] * D[0]) * ir;
     c[4] += (D[4] - c[4] * D[0]) * ir;
-    c[1] = fmax((E + D[1]) * (gam - real(1)), pmin);
+    c[1] = fmax(fma(D[1], fac, E) * (gam - real(1)), pmin);
     c[0] = rn;
 }
 
@@ -358,23 +392,27 @@ __device__ __forceinline__ void source_cell(const SphK<real>& a, const PlanetS<r
                                             real dt, real& un, real& vn, real& wn);
 
 // ----------------------------------------------------------------- sweeps
-// DIR 0: radius (rows (j, k), segments of a.tx cells, one thread per slot);
-// 1: azimuth (R radii x SPH_TY cells per block); 2: polar angle (R radii x
-// the whole column).  DIR 0 with hkick != 0 first applies the step's first
-// half kick (the source terms at t with mdt = 0 over hkick = dt/2, planet pl)
-// to every interior cell it loads, in place of a source-term pass; the block
-// has a thread per slot, so each thread keeps its own cell's kicked state in
-// registers for the update.
+// DIR 0: radius (a.xr rows (j, k) x a segment of a.tx cells, one thread per
+// slot); 1: azimuth (R radii x SPH_TY cells per block); 2: polar angle (R
+// radii x the whole column).  DIR 0 with hkick != 0 first applies the step's
+// first half kick (the source terms at t with mdt = 0 over hkick = dt/2,
+// planet pl) to every interior cell it loads, in place of a source-term pass;
+// the block has a thread per slot, so each thread keeps its own cell's kicked
+// state in registers for the update.  The azimuthal sweep takes the cell it
+// updates from LDS, which holds every field as loaded, the polar sweep all but
+// vp.  Seven waves per SIMD are asked for where they cost no spill (PPM4 in
+// FP32, 72 registers for 79: radial sweep of a 101x190x33 disk 27.2 -> 24.9 us;
+// PEM4 spills 100 bytes a lane there, 1021 -> 1094 us on the 384x1536x64 disk).
 template <typename real, int DIR, int RECON>
-__global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<real> a, real dt, PlanetS<real> pl,
-                                                                         int planet, real hkick) {
+__global__ __launch_bounds__(SPH_BT2, RECON == 6 && sizeof(real) == 4 ? 7 : 1) void k3_sweep(
+    SphK<real> a, real dt, PlanetS<real> pl, int planet, real hkick) {
     extern __shared__ __align__(16) unsigned char sm_raw[];
     real* sm = reinterpret_cast<real*>(sm_raw);
-    constexpr int R = DIR == 0 ? 1 : SPH_R;
+    constexpr int R = DIR == 0 ? 1 : SPH_R;   // LDS distance of neighbours along the sweep
     const int BT = DIR == 0 ? (int)blockDim.x : SPH_BT2;
     const int L = DIR == 0 ? a.tx : DIR == 1 ? SPH_TY : a.nz;
     const int S = L + 2 * NPAD;
-    const int RS = R * S;         // at most 2 BT (checked by the host)
+    const int RS = (DIR == 0 ? a.xr : R) * S;   // at most BT, for DIR 2 2 BT (the host's choice of tile)
     real* raw = sm;              // [5][RS]
     real* TLs = raw + NF * RS;   // state left of each cell's right edge
     real* TRs = TLs + NF * RS;   // state right of each cell's left edge
@@ -384,45 +422,60 @@ __global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<re
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const size_t N = a.N;
 
-    // tile of this block
-    int i0 = 0, j0 = 0, k0 = 0;   // first interior cell of the segment / first row
+    // tile of this block: i0, j0, k0 its first interior cell; cells are
+    // addressed from c0 (uniform over the block) by a 32-bit lane offset
+    int i0 = 0, j0 = 0, k0 = 0;
+    size_t c0 = 0;
     const int bt = xcd_tile(blockIdx.x, gridDim.x);
+    // DIR 0: this thread's slot, row and polar layer; rows are consecutive in
+    // memory whatever their layer
+    int s0 = 0, jr = 0, kr = 0;
+    unsigned ro = 0;
+    bool in_row = true;
     if (DIR == 0) {
         const int ntx = (nx + a.tx - 1) / a.tx;
-        const int row = bt / ntx;
-        i0 = (bt - row * ntx) * a.tx;
-        j0 = row % ny;
-        k0 = row / ny;
+        const int rg = bt / ntx;
+        i0 = (bt - rg * ntx) * a.tx;
+        const int r = (t * a.xm) >> 20;   // t / S
+        s0 = t - r * S;
+        const int row = rg * a.xr + r;
+        in_row = r < a.xr && row < ny * nz;
+        kr = in_row ? row / ny : 0;
+        jr = in_row ? row - kr * ny : 0;
+        ro = (unsigned)(r * nx);
+        c0 = (size_t)rg * a.xr * nx;
     } else if (DIR == 1) {
         const int nty = (ny + SPH_TY - 1) / SPH_TY, nig = (nx + R - 1) / R;
         const int rest = bt / nig;
         i0 = (bt - rest * nig) * R;
         j0 = (rest % nty) * SPH_TY;
         k0 = rest / nty;
+        c0 = (size_t)k0 * nx * ny;
     } else {
         const int nig = (nx + R - 1) / R;
         i0 = (bt % nig) * R;
         j0 = bt / nig;
     }
+    auto get = [&](int f, unsigned o) { return ld_off(gmem(a.in) + (f * N + c0), o * (unsigned)sizeof(real)); };
 
     // ---- load (with the sweep's field rotation and angular momenta)
     real own[NF] = {};   // DIR 0: this thread's cell as loaded (and kicked)
     for (int e = t; e < RS; e += BT) {
-        const int s = e / R, r = e - (e / R) * R;
+        const int s = DIR == 0 ? s0 : e / R, r = e - (e / R) * R;
         real v[NF] = {real(1), real(1), real(0), real(0), real(0)};
         if (DIR == 0) {
             const int i = i0 + s - NPAD, ip = i + NPAD;
-            if (i < nx + NPAD) {
-                const int k = k0;
+            if (in_row && i < nx + NPAD) {
                 real vp;
                 if (i >= 0 && i < nx) {
-                    const size_t c = (size_t)i + (size_t)nx * ((size_t)j0 + (size_t)ny * k);
-                    v[0] = a.in[c]; v[1] = a.in[N + c]; v[2] = a.in[2 * N + c];
-                    vp = a.in[3 * N + c]; v[4] = a.in[4 * N + c];
+                    const unsigned o = ro + (unsigned)i;
+                    v[0] = get(0, o); v[1] = get(1, o); v[2] = get(2, o); vp = get(3, o); v[4] = get(4, o);
                     if (hkick != real(0)) {
-                        const real visr = a.vis ? a.vis[c] : real(0), visp = a.vis ? a.vis[N + c] : real(0);
+                        const PG_GLOBAL real* vis = gmem(a.vis) + c0;
+                        const real visr = a.vis ? ld_off(vis, o * (unsigned)sizeof(real)) : real(0);
+                        const real visp = a.vis ? ld_off(vis + N, o * (unsigned)sizeof(real)) : real(0);
                         real un, vn, wn;
-                        source_cell(a, pl, planet != 0, ip, k + NPAD, j0, v[0], v[2], vp, v[4], visr, visp, real(0),
+                        source_cell(a, pl, planet != 0, ip, kr + NPAD, jr, v[0], v[2], vp, v[4], visr, visp, real(0),
                                     hkick, un, vn, wn);
                         v[2] = un;
                         vp = vn;
@@ -431,23 +484,22 @@ __global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<re
                     own[0] = v[0]; own[1] = v[1]; own[2] = v[2]; own[3] = vp; own[4] = v[4];
                 } else {
                     const int g = i < 0 ? ip : ip - nx;
-                    const real* xg = a.xg + (size_t)g * nz + k;
+                    const real* xg = a.xg + (size_t)g * nz + kr;
                     v[0] = xg[0]; v[1] = xg[6 * nz]; v[2] = xg[12 * nz]; vp = xg[18 * nz]; v[4] = xg[24 * nz];
                 }
                 const real rad = a.xc[ip];
-                const real rcyl = rad * a.sinz[k + NPAD];
-                v[3] = (vp + a.vbg[(size_t)k * (nx + 2 * NPAD) + ip]) * rcyl;   // v R_cyl
-                v[4] *= rad;                                                    // w r
+                const real rcyl = rad * a.sinz[kr + NPAD];
+                v[3] = (vp + a.vbg[(size_t)kr * (nx + 2 * NPAD) + ip]) * rcyl;   // v R_cyl
+                v[4] *= rad;                                                     // w r
             }
         } else if (DIR == 1) {
             const int i = i0 + r;
             if (i < nx) {
-                const int j = wrapi(j0 + s - NPAD, ny);
-                const size_t c = (size_t)i + (size_t)nx * ((size_t)j + (size_t)ny * k0);
-                v[0] = a.in[c]; v[1] = a.in[N + c];
-                v[2] = a.in[3 * N + c];   // normal: vp = v - rot - R_cyl Omega
-                v[3] = a.in[4 * N + c];   // w
-                v[4] = a.in[2 * N + c];   // u
+                const unsigned o = (unsigned)i + (unsigned)nx * (unsigned)wrapi(j0 + s - NPAD, ny);
+                v[0] = get(0, o); v[1] = get(1, o);
+                v[2] = get(3, o);   // normal: vp = v - rot - R_cyl Omega
+                v[3] = get(4, o);   // w
+                v[4] = get(2, o);   // u
             }
         } else {
             const int i = i0 + r;
@@ -469,7 +521,7 @@ __global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<re
 
     // ---- per cell: parameters and the two traced states
     for (int e = t; e < RS; e += BT) {
-        const int s = e / R, r = e - (e / R) * R;
+        const int s = DIR == 0 ? s0 : e / R, r = e - (e / R) * R;
         if (s < 2 || s > S - 3) continue;
         real idx, dts;
         const real* w;
@@ -525,11 +577,17 @@ __global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<re
 
     // ---- per interface s (between cells s-1 and s): HLLC; every thread
     // reads its traced states before any flux overwrites them
-    real Fr[2][NF + 2];
+    constexpr int NI = DIR == 2 ? 2 : 1;   // interfaces per thread, at most
+    real Fr[NI][NF + 2];
+    auto iface = [&](int m, int& e) {
+        e = t + m * BT;
+        const int s = DIR == 0 ? s0 : e / R;
+        return e < RS && s >= NPAD && s <= S - NPAD && !(DIR == 0 && i0 + s > nx + 2 * NPAD - 3);
+    };
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const int e = t + m * BT, s = e / R;
-        if (e >= RS || s < NPAD || s > S - NPAD || (DIR == 0 && i0 + s > nx + 2 * NPAD - 3)) continue;
+    for (int m = 0; m < NI; ++m) {
+        int e;
+        if (!iface(m, e)) continue;
         real Ls[NF], Rs[NF];
         for (int f = 0; f < NF; ++f) {
             Ls[f] = TLs[f * RS + e - R];
@@ -540,9 +598,9 @@ __global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<re
     }
     __syncthreads();
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        const int e = t + m * BT, s = e / R;
-        if (e >= RS || s < NPAD || s > S - NPAD || (DIR == 0 && i0 + s > nx + 2 * NPAD - 3)) continue;
+    for (int m = 0; m < NI; ++m) {
+        int e;
+        if (!iface(m, e)) continue;
         for (int f = 0; f < NF; ++f) TLs[f * RS + e] = Fr[m][f];
         TRs[e] = Fr[m][NF];
         TRs[RS + e] = Fr[m][NF + 1];
@@ -551,24 +609,30 @@ __global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<re
 
     // ---- per cell: flux and source differences (net_source, riemann.cu:40-87), update
     for (int e = t; e < RS; e += BT) {
-        const int s = e / R, r = e - (e / R) * R;
+        const int s = DIR == 0 ? s0 : e / R, r = e - (e / R) * R;
         if (s < NPAD || s >= S - NPAD) continue;
-        int i, j, k;
+        int i, k;
+        unsigned o = 0;   // the cell from c0 (DIR 2: from its own 64-bit index)
+        size_t c = 0;
         real g0, g1, fac;
         if (DIR == 0) {
-            i = i0 + s - NPAD; j = j0; k = k0;
-            if (i >= nx) continue;
+            i = i0 + s - NPAD; k = kr;
+            if (i >= nx || !in_row) continue;
+            o = ro + (unsigned)i;
             g0 = a.xa[i + NPAD] * a.xa[i + NPAD];
             g1 = a.xa[i + NPAD + 1] * a.xa[i + NPAD + 1];
             fac = FM<real>::div(dt, a.xv[i + NPAD]);
         } else if (DIR == 1) {
-            i = i0 + r; j = j0 + s - NPAD; k = k0;
+            const int j = j0 + s - NPAD;
+            i = i0 + r; k = k0;
             if (i >= nx || j >= ny) continue;
+            o = (unsigned)i + (unsigned)nx * (unsigned)j;
             g0 = g1 = real(1);
             fac = FM<real>::div(dt, a.dy * (a.xc[i + NPAD] * a.sinz[k + NPAD]));
         } else {
-            i = i0 + r; j = j0; k = s - NPAD;
+            i = i0 + r; k = s - NPAD;
             if (i >= nx) continue;
+            c = (size_t)i + (size_t)nx * ((size_t)j0 + (size_t)ny * k);
             g0 = a.sza[s];
             g1 = a.sza[s + 1];
             fac = FM<real>::div(dt, a.zv[s] * a.xc[i + NPAD]);
@@ -584,34 +648,36 @@ __global__ __launch_bounds__(DIR == 0 ? SPH_BTX : SPH_BT2) void k3_sweep(SphK<re
         const real de = real(0.5) * (p0s + p1s) * (TRs[RS + e] * g0 - TRs[RS + e + R] * g1);
         real D[NF];
         D[0] = (F0[0] * g0 - F1[0] * g1) * fac;
-        D[1] = (F0[RS] * g0 - F1[RS] * g1 + de) * fac;
+        D[1] = F0[RS] * g0 - F1[RS] * g1 + de;
         D[2] = (F0[2 * RS] * g0 - F1[2 * RS] * g1 + du) * fac;
         D[3] = (F0[3 * RS] * g0 - F1[3 * RS] * g1) * fac;
         D[4] = (F0[4 * RS] * g0 - F1[4 * RS] * g1) * fac;
-        const size_t c = (size_t)i + (size_t)nx * ((size_t)j + (size_t)ny * k);
-        const real vb = a.vbg[(size_t)k * (nx + 2 * NPAD) + i + NPAD];
-        real U[NF];   // changes of mass, internal energy, u, vp, w momenta
+        real U[NF];      // changes of mass, internal energy, u, vp, w momenta
+        real cell[NF];   // the cell before the sweep
+        const real* x = raw + e;
+        U[0] = D[0]; U[1] = D[1];
         if (DIR == 0) {
             const real rad = a.xc[i + NPAD], rcyl = rad * a.sinz[k + NPAD];
-            U[0] = D[0]; U[1] = D[1]; U[2] = D[2];
-            U[3] = FM<real>::div(D[3], rcyl) - vb * D[0];
+            U[2] = D[2];
+            U[3] = FM<real>::div(D[3], rcyl) - a.vbg[(size_t)k * (nx + 2 * NPAD) + i + NPAD] * D[0];
             U[4] = FM<real>::div(D[4], rad);
+            for (int f = 0; f < NF; ++f) cell[f] = own[f];
         } else if (DIR == 1) {
-            U[0] = D[0]; U[1] = D[1];
             U[3] = D[2];   // vp momentum (the frame term is the background's)
             U[4] = D[3];
             U[2] = D[4];
+            cell[0] = x[0]; cell[1] = x[RS]; cell[3] = x[2 * RS]; cell[4] = x[3 * RS]; cell[2] = x[4 * RS];
         } else {
-            const real rcyl = a.xc[i + NPAD] * a.sinz[s];
-            U[0] = D[0]; U[1] = D[1];
             U[4] = D[2];
             U[2] = D[3];
-            U[3] = FM<real>::div(D[4], rcyl) - vb * D[0];
+            U[3] = FM<real>::div(D[4], a.xc[i + NPAD] * a.sinz[s]) - a.vbg[(size_t)k * (nx + 2 * NPAD) + i + NPAD] * D[0];
+            cell[0] = x[0]; cell[1] = x[RS]; cell[4] = x[2 * RS]; cell[2] = x[3 * RS]; cell[3] = a.in[3 * N + c];
         }
-        real cell[NF];
-        for (int f = 0; f < NF; ++f) cell[f] = DIR == 0 ? own[f] : a.in[f * N + c];
-        update_cell(cell, U, a.gam);
-        for (int f = 0; f < NF; ++f) a.out[f * N + c] = cell[f];
+        update_cell(cell, U, fac, a.gam);
+        for (int f = 0; f < NF; ++f) {
+            if (DIR == 2) a.out[f * N + c] = cell[f];
+            else *(PG_GLOBAL real*)((PG_GLOBAL char*)(gmem(a.out) + (f * N + c0)) + o * (unsigned)sizeof(real)) = cell[f];
+        }
     }
 }
 
@@ -673,7 +739,7 @@ __global__ __launch_bounds__(SPH_BT) void k3_orbadv(SphK<real> a, double dt, int
         const real dte = FM<real>::div((real)dt, a.xc[i + NPAD] * a.sinz[k0 + NPAD]);
         const bool up = speed > real(0);
         const int cs = up ? s - 1 : s;
-        const real q = lim01(fabs(speed) * dte * a.idy);
+        const real q = up ? edge_fraction<1>(speed * dte * a.idy) : edge_fraction<-1>(-speed * dte * a.idy);
         const real* x = raw + cs * R + r;
         // the upwind cell's mean next to this interface: its right edge, or
         // its left one; the first is the second of the mirrored profile,
@@ -686,11 +752,9 @@ __global__ __launch_bounds__(SPH_BT) void k3_orbadv(SphK<real> a, double dt, int
             const real l = P[f].sL;
             P[f].sL = up ? -P[f].sR : l;
             P[f].sR = up ? -l : P[f].sR;
-            P[f].sS = up ? -P[f].sS : P[f].sS;
             P[f].zl = P[f].zl != up;
         }
-        edge_means<RECON, -1, NF, real>(q, {&P[0], &P[1], &P[2], &P[3], &P[4]}, D);
-        for (int f = 0; f < NF; ++f) D[f] += P[f].a;
+        edge_means<RECON, -1, NF>(q, P, D);
         FX[e] = D[0] * speed;
         FX[RS + e] = D[1] * speed;
         for (int f = 2; f < NF; ++f) FX[f * RS + e] = D[f] * D[0] * speed;
@@ -1099,15 +1163,18 @@ SphK<real> kargs(Sph* s, int in, int out) {
     a.idy = (real)(1.0 / dy);
     a.dy_d = dy;
     a.gam = (real)s->P.gam;
-    a.tx = sph_tx(s->nx);
+    const RadialTile rt = radial_tile(s->nx, (long)s->ny * s->nz, (int)sizeof(real));
+    a.tx = rt.tx;
+    a.xr = rt.xr;
+    a.xm = (1 << 20) / (rt.tx + 2 * NPAD) + 1;
     return a;
 }
 
 template <typename real>
-size_t sweep_lds(int dir, int nx, int nz) {
-    const int R = dir == 0 ? 1 : SPH_R;
-    const int L = dir == 0 ? sph_tx(nx) : dir == 1 ? SPH_TY : nz;
-    return (size_t)(3 * NF) * R * (L + 2 * NPAD) * sizeof(real);
+size_t sweep_lds(const SphK<real>& a, int dir) {
+    const int rows = dir == 0 ? a.xr : SPH_R;
+    const int L = dir == 0 ? a.tx : dir == 1 ? SPH_TY : a.nz;
+    return (size_t)(3 * NF) * rows * (L + 2 * NPAD) * sizeof(real);
 }
 
 // launch timing (profiling): events around one launch, synchronous
@@ -1160,16 +1227,16 @@ int launch_sweep(Sph* s, int dir, int in, int out, double dt, const Body* kick =
     }
     const int planet = kick && s->P.n_planet > 0 ? 1 : 0;
     const real hk = kick ? (real)hkick : real(0);
-    const size_t lds = sweep_lds<real>(dir, s->nx, s->nz);
+    const size_t lds = sweep_lds<real>(a, dir);
     unsigned nb;
-    if (dir == 0) nb = (unsigned)(((s->nx + a.tx - 1) / a.tx) * s->ny * s->nz);
+    if (dir == 0) nb = (unsigned)(((s->nx + a.tx - 1) / a.tx) * ((s->ny * s->nz + a.xr - 1) / a.xr));
     else if (dir == 1) nb = (unsigned)(((s->ny + SPH_TY - 1) / SPH_TY) * ((s->nx + SPH_R - 1) / SPH_R) * s->nz);
     else nb = (unsigned)(((s->nx + SPH_R - 1) / SPH_R) * s->ny);
     Timed tm(s, kSphKernels[dir]);
     const bool pem = s->P.recon_flag == 5;
 #define SPH_SWEEP(D)                                                                                   \
     do {                                                                                               \
-        const int bt = D == 0 ? sph_bx(s->nx) : SPH_BT2;                                               \
+        const int bt = D == 0 ? (a.xr * (a.tx + 2 * NPAD) + 63) / 64 * 64 : SPH_BT2;                                               \
         if (pem) {                                                                                     \
             SPH_TRY(allow_lds(k3_sweep<real, D, 5>, lds));                                             \
             hipLaunchKernelGGL((k3_sweep<real, D, 5>), dim3(nb), dim3(bt), lds, s->stream, a, (real)dt, pl, \
