@@ -30,6 +30,7 @@
 
 #include "../../include/penguin_amd.h"
 #include "pg_device.h"
+#include "pg_frame.h"
 #include "pg_internal.h"
 #include "pg_launch.h"
 #include "pg_sph.h"
@@ -332,6 +333,7 @@ struct Group {
     // pinned host staging for results read back after a run (the step sizes)
     double* stage = nullptr;
     size_t stage_bytes = 0;
+    FrameBuf frame;              // pinned pieces of a state being read back
 
     int par() const { return gpar | (dpar << 1); }
     int ndisk() const { return (int)disks.size(); }
@@ -810,6 +812,7 @@ void group_release(Group& g) {
     if (g.stage) (void)hipHostFree(g.stage);
     g.stage = nullptr;
     g.stage_bytes = 0;
+    g.frame.release();
     if (g.ev_a) (void)hipEventDestroy(g.ev_a);
     if (g.ev_b) (void)hipEventDestroy(g.ev_b);
     if (g.stream) (void)hipStreamDestroy(g.stream);
@@ -1147,36 +1150,54 @@ int group_run(Group& g, int nsteps, double* t_io, double* dt_io, double* dts, in
 }
 
 // ------------------------------------------------------------ state I/O
-int disk_get_state(Group& g, int k, double* gas, double* dust) {
-    DiskDev* h = g.disks[k];
-    const size_t N = h->N;
-    const int nx = h->nx;
-    std::vector<double> gv, dv;
-    int rc;
-    if (gas) {
-        if ((rc = download(h->prec, g.stream, h->gas[g.gpar], gv, 3 * N))) return rc;
-        for (size_t o = 0; o < N; ++o) {
-            int ip = (int)(o % nx) + NPAD;
-            double rho = h->rho_bg[o % nx] + gv[o];
-            gas[o] = rho;
-            gas[N + o] = tabv(h, T_CS2, ip) * rho;
-            gas[2 * N + o] = gv[N + o];
-            gas[3 * N + o] = tabv(h, T_VBG, ip) + gv[2 * N + o];
-            gas[4 * N + o] = 0.0;
-        }
-    }
-    if (dust) {
-        if (!h->P.dust_flag) return fail(PG_E_STATE, "the disk has no dust");
-        if ((rc = download(h->prec, g.stream, h->dust[g.dpar], dv, 3 * N))) return rc;
-        for (size_t o = 0; o < N; ++o) {
-            int ip = (int)(o % nx) + NPAD;
-            dust[o] = dv[o];
-            dust[N + o] = dv[N + o];
-            dust[2 * N + o] = tabv(h, T_VBG, ip) + dv[2 * N + o];
-            dust[3 * N + o] = 0.0;
-        }
-    }
+template <typename real>
+int get_state_t(Group& g, const DiskDev* h, double* gas, double* dust) {
+    const size_t N = h->N, nx = h->nx, ny = h->ny;
+    const double* rb = h->rho_bg.data();
+    const double* cs2 = h->tabh.data() + (size_t)T_CS2 * h->tab_stride + NPAD;
+    const double* vbg = h->tabh.data() + (size_t)T_VBG * h->tab_stride + NPAD;
+    if (gas)
+        HIP_TRY(read_frame(g.frame, g.stream, h->gas[g.gpar], N * sizeof(real), 3, ny, nx, sizeof(real),
+                           [=](const char* src, size_t m, size_t r0, size_t r1) {
+            for (size_t r = r0; r < r1; ++r, src += nx * sizeof(real)) {
+                const real* f0 = (const real*)src;
+                const real* f1 = (const real*)(src + m);
+                const real* f2 = (const real*)(src + 2 * m);
+                double* o = gas + r * nx;
+                for (size_t i = 0; i < nx; ++i) {
+                    const double rho = rb[i] + (double)f0[i];
+                    o[i] = rho;
+                    o[N + i] = cs2[i] * rho;
+                }
+                for (size_t i = 0; i < nx; ++i) o[2 * N + i] = (double)f1[i];
+                for (size_t i = 0; i < nx; ++i) o[3 * N + i] = vbg[i] + (double)f2[i];
+                for (size_t i = 0; i < nx; ++i) o[4 * N + i] = 0.0;
+            }
+        }));
+    if (dust)
+        HIP_TRY(read_frame(g.frame, g.stream, h->dust[g.dpar], N * sizeof(real), 3, ny, nx, sizeof(real),
+                           [=](const char* src, size_t m, size_t r0, size_t r1) {
+            for (size_t r = r0; r < r1; ++r, src += nx * sizeof(real)) {
+                const real* f0 = (const real*)src;
+                const real* f1 = (const real*)(src + m);
+                const real* f2 = (const real*)(src + 2 * m);
+                double* o = dust + r * nx;
+                for (size_t i = 0; i < nx; ++i) o[i] = (double)f0[i];
+                for (size_t i = 0; i < nx; ++i) o[N + i] = (double)f1[i];
+                for (size_t i = 0; i < nx; ++i) o[2 * N + i] = vbg[i] + (double)f2[i];
+                for (size_t i = 0; i < nx; ++i) o[3 * N + i] = 0.0;
+            }
+        }));
     return PG_OK;
+}
+
+int disk_get_state(Group& g, int k, double* gas, double* dust) {
+    const DiskDev* h = g.disks[k];
+    if (dust && !h->P.dust_flag) {
+        const int rc = gas ? disk_get_state(g, k, gas, nullptr) : PG_OK;
+        return rc ? rc : fail(PG_E_STATE, "the disk has no dust");
+    }
+    return h->prec == 8 ? get_state_t<double>(g, h, gas, dust) : get_state_t<float>(g, h, gas, dust);
 }
 
 int disk_set_state(Group& g, int k, const double* gas, const double* dust) {

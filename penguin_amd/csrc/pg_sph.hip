@@ -41,6 +41,7 @@
 
 #include "../../include/penguin_amd.h"
 #include "pg_device.h"
+#include "pg_frame.h"
 #include "pg_internal.h"
 #include "pg_sph.h"
 
@@ -1122,6 +1123,7 @@ struct Sph {
     double* dtab = nullptr;     // FP64 tables: rot, rcyl
     void* rate = nullptr;
     void* rate_h = nullptr;     // pinned
+    FrameBuf frame;             // pinned pieces of a state being read back
     size_t tab_off[16] = {0};
     std::vector<double> xa, xv, ya, yv, za, zv, vbg, rot, rcyl;
     std::vector<double> xgh;    // radial ghost states (rho, p, u, v, w) [field][ghost 0..5][polar k], FP64
@@ -1484,19 +1486,20 @@ int put_state(Sph* s, const double* gas) {
 }
 template <typename real>
 int get_state(Sph* s, double* gas) {
-    const size_t N = s->N;
-    const int nx = s->nx, ny = s->ny, nxe = nx + 2 * NPAD;
-    std::vector<real> h((size_t)NF * N);
-    SPH_TRY(hipMemcpyAsync(h.data(), s->st[0], h.size() * sizeof(real), hipMemcpyDeviceToHost, s->stream));
-    SPH_TRY(hipStreamSynchronize(s->stream));
-    for (size_t c = 0; c < N; ++c) {
-        const int i = (int)(c % nx), k = (int)(c / nx / ny);
-        gas[c] = (double)h[c];
-        gas[N + c] = (double)h[N + c];
-        gas[2 * N + c] = (double)h[2 * N + c];
-        gas[3 * N + c] = (double)h[3 * N + c] + s->vbg[(size_t)k * nxe + i + NPAD];
-        gas[4 * N + c] = (double)h[4 * N + c];
-    }
+    const size_t N = s->N, nx = s->nx, ny = s->ny, nxe = nx + 2 * NPAD;
+    const double* vbg = s->vbg.data();
+    SPH_TRY(read_frame(s->frame, s->stream, s->st[0], N * sizeof(real), NF, ny * s->nz, nx, sizeof(real),
+                       [=](const char* src, size_t m, size_t r0, size_t r1) {
+        for (size_t r = r0; r < r1; ++r, src += nx * sizeof(real)) {
+            const double* vb = vbg + r / ny * nxe + NPAD;
+            for (int f = 0; f < NF; ++f) {
+                const real* x = (const real*)(src + f * m);
+                double* o = gas + f * N + r * nx;
+                if (f == 3) for (size_t i = 0; i < nx; ++i) o[i] = (double)x[i] + vb[i];
+                else for (size_t i = 0; i < nx; ++i) o[i] = (double)x[i];
+            }
+        }
+    }));
     return PG_OK;
 }
 
@@ -1622,6 +1625,7 @@ void sph_destroy(Sph* s) {
     if (s->dtab) (void)hipFree(s->dtab);
     if (s->rate) (void)hipFree(s->rate);
     if (s->rate_h) (void)hipHostFree(s->rate_h);
+    s->frame.release();
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
 }
