@@ -401,11 +401,12 @@ __device__ __forceinline__ void source_cell(const SphK<real>& a, const PlanetS<r
 // the block has a thread per slot, so each thread keeps its own cell's kicked
 // state in registers for the update.  The azimuthal sweep takes the cell it
 // updates from LDS, which holds every field as loaded, the polar sweep all but
-// vp.  Seven waves per SIMD are asked for where they cost no spill (PPM4 in
-// FP32, 72 registers for 79: radial sweep of a 101x190x33 disk 27.2 -> 24.9 us;
-// PEM4 spills 100 bytes a lane there, 1021 -> 1094 us on the 384x1536x64 disk).
+// vp.  PPM4 is held to seven waves per SIMD in FP32 (72 registers for 79: radial
+// sweep of a 101x190x33 disk 27.2 -> 24.9 us) and to four, two blocks per CU, in
+// FP64 (128 for 136; 40x64x16 step 71.4 -> 69.1 us); PEM4 would spill 100 bytes a
+// lane (1021 -> 1094 us on the 384x1536x64 disk).
 template <typename real, int DIR, int RECON>
-__global__ __launch_bounds__(SPH_BT2, RECON == 6 && sizeof(real) == 4 ? 7 : 1) void k3_sweep(
+__global__ __launch_bounds__(SPH_BT2, RECON != 6 ? 1 : sizeof(real) == 4 ? 7 : 4) void k3_sweep(
     SphK<real> a, real dt, PlanetS<real> pl, int planet, real hkick) {
     extern __shared__ __align__(16) unsigned char sm_raw[];
     real* sm = reinterpret_cast<real*>(sm_raw);
