@@ -794,7 +794,7 @@ __device__ __forceinline__ void src_adj_cell(const DiskArgs<real>& d, int mode, 
     const PlanetK& pk = mode == 0 ? d.ctl->pk0 : d.ctl->pk1;
     const real iR = TAB(T_IR, ip), vbg = TAB(T_VBG, ip);
     real px = real(0), py = real(0);
-    if (d.n_planet > 0) planet_acc(pk, d.phitab + 4 * j, TAB(T_XC, ip), px, py);
+    if (d.n_planet > 0) planet_acc(pk, (const PG_CONST real*)d.phitab + 4 * j, TAB(T_XC, ip), px, py);
     const real irho = FM<real>::rcp(rho);
     if (!d.visc) { Vr = real(0); Vp = real(0); }
     const real vy = Vp * irho;

@@ -33,6 +33,11 @@ __device__ __forceinline__ const PG_GLOBAL T* gmem(const T* p) { return (const P
 template <typename T>
 __device__ __forceinline__ PG_GLOBAL T* gmem(T* p) { return (PG_GLOBAL T*)p; }
 
+// Memory that no thread writes while the kernel runs (the control block and the
+// descriptors in the passes of a step, the tables): uniform reads through this
+// view go to scalar registers.
+#define PG_CONST __attribute__((address_space(4)))
+
 // Load at a uniform base plus an unsigned 32-bit byte offset: the form the
 // scalar-base global load takes, so no 64-bit address arithmetic per load.
 template <typename T>
@@ -64,6 +69,15 @@ template <> struct FM<double> {
 };
 
 // ---------------------------------------------------------------- helpers
+// A product that is rounded before it is added to anything: where a sum of two
+// products could contract either into a fused multiply-add, the choice would
+// be the compiler's in each tile variant, and the variants' results would
+// differ in the last bit.
+template <typename real>
+PG_HD real mul_rn(real a, real b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
 template <typename real>
 PG_HD real lim01(real a) {  // solve.cu:14-17
     return fmin(fmax(a, real(0)), real(1));
@@ -618,19 +632,48 @@ __device__ __forceinline__ int wrap(int j, int n) {
 // angle phi_j from the tabulated sin/cos of phi_j and phi_j/2 and the
 // planet's (sin, cos) of phi_p and phi_p/2.  The squared distance is written
 // without cancellation: (R - a)^2 + 4 a R sin^2((phi - phi_p)/2) + rs^2.
-template <typename real>
-__device__ __forceinline__ void planet_acc(const PlanetK& pk, const real* pt, real R, real& ax, real& ay) {
+template <typename real, typename PK>
+__device__ __forceinline__ void planet_acc(const PK& pk, const PG_CONST real* pt, real R, real& ax, real& ay) {
     const real sp = (real)pk.sphi, cp = (real)pk.cphi, shp = (real)pk.shphi, chp = (real)pk.chphi;
-    const real s = pt[0] * cp - pt[1] * sp;      // sin(phi - phi_p)
-    const real c = pt[1] * cp + pt[0] * sp;      // cos(phi - phi_p)
-    const real h = pt[2] * chp - pt[3] * shp;    // sin((phi - phi_p)/2)
+    // sums of two products in a written order, so that every kernel variant
+    // rounds them alike (see mul_rn)
+    const real s = fma(pt[0], cp, -(pt[1] * sp));      // sin(phi - phi_p)
+    const real c = fma(pt[1], cp, pt[0] * sp);         // cos(phi - phi_p)
+    const real h = fma(pt[2], chp, -(pt[3] * shp));    // sin((phi - phi_p)/2)
     const real px = (real)pk.x, m = (real)pk.m, rs = (real)pk.rs;
-    const real Rp2 = (R - px) * (R - px) + real(4) * px * R * h * h + rs * rs;
+    const real Rp2 = fma(R - px, R - px, fma(real(4) * px * R * h, h, rs * rs));
     const real iRp = FM<real>::rsqrt(Rp2);
     const real k = iRp * iRp * iRp;
     const real ind = (real)pk.m_over_x2;
-    ax = -m * (R - px * c) * k - c * ind;
-    ay = -m * px * s * k + s * ind;
+    ax = fma(-m * fma(-px, c, R), k, -(c * ind));
+    ay = fma(-m * px * s, k, s * ind);
+}
+
+// What the source terms read of the step, in the storage precision: dt, dt/2
+// and the planet at t (late = 0) or t + dt (late = 1), in scalar registers.
+// (Converted from FP64 in vector registers for every cell, these ten constants
+// were 20 of the x sweep's 525 instructions: 1024x3072 gas and dust step 222 ->
+// 204 us, in FP64 552 -> 524, 24 disks 372 -> 348 us, together with the x
+// sweeps' table registers no longer cleared.)
+template <typename real>
+struct StepView {
+    real dt, h;
+    PlanetKT<real> pk;
+};
+template <typename real>
+__device__ __forceinline__ StepView<real> step_view(const StepCtl* ctl, int late);
+template <>
+__device__ __forceinline__ StepView<float> step_view<float>(const StepCtl* ctl, int late) {
+    const PG_CONST StepCtl* c = (const PG_CONST StepCtl*)ctl;
+    const PG_CONST PlanetKT<float>* k = late ? &c->pf1 : &c->pf0;
+    return {c->dt_f, c->h_f, {k->m, k->x, k->rs, k->m_over_x2, k->sphi, k->cphi, k->shphi, k->chphi}};
+}
+template <>
+__device__ __forceinline__ StepView<double> step_view<double>(const StepCtl* ctl, int late) {
+    const PG_CONST StepCtl* c = (const PG_CONST StepCtl*)ctl;
+    const PG_CONST PlanetK* k = late ? &c->pk1 : &c->pk0;
+    const double dt = c->dt;
+    return {dt, 0.5 * dt, {k->m, k->x, k->rs, k->m_over_x2, k->sphi, k->cphi, k->shphi, k->chphi}};
 }
 
 }  // namespace pg

@@ -650,6 +650,7 @@ int disk_create(const pg_params& P, hipStream_t s, DiskDev** out) {
     c.planet0 = b0;
     c.planet1 = b0;
     c.pk0 = c.pk1 = planet_kernel_view(b0);
+    c.pf0 = c.pf1 = planet_kernel_view_f(c.pk0);
     c.end_time = P.end_time;
     if (hipMemcpyAsync(h->ctl, h->ctl_host, sizeof(StepCtl), hipMemcpyHostToDevice, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
@@ -2191,6 +2192,7 @@ int pg_sources(pg_handle* h, double t_planet, double mdt, double dt, int inplace
     if ((rc = pull_ctl(g))) return rc;
     c.planet1 = c.planet0;
     c.pk1 = c.pk0;
+    c.pf1 = c.pf0;
     if ((rc = push_ctl(g))) return rc;
     hipError_t e = g.prec == 8 ? Launch<double>::sources(g.ls<double>(), g.par(), mode, 0, 0, g.stream)
                                : Launch<float>::sources(g.ls<float>(), g.par(), mode, 0, 0, g.stream);
@@ -2673,6 +2675,7 @@ static int adjoint_pass(pg_handle* h, int pass, double t, double dt, const doubl
         if ((rc = pull_ctl(g))) return rc;
         c.planet1 = c.planet0;
         c.pk1 = c.pk0;
+        c.pf1 = c.pf0;
         if ((rc = push_ctl(g))) return rc;
     }
     size_t scratch = 0;

@@ -51,9 +51,11 @@ struct Body {
 
 // A planet as the source kernel uses it: mass, orbital radius, softening,
 // m/x^2 (indirect term) and the sine/cosine of its angle and half angle.
-struct PlanetK {
-    double m, x, rs, m_over_x2, sphi, cphi, shphi, chphi;
+template <typename T>
+struct PlanetKT {
+    T m, x, rs, m_over_x2, sphi, cphi, shphi, chphi;
 };
+using PlanetK = PlanetKT<double>;
 
 // What the source kernel needs of a planet, precomputed once per step.
 __host__ __device__ inline PlanetK planet_kernel_view(const Body& b) {
@@ -69,7 +71,14 @@ __host__ __device__ inline PlanetK planet_kernel_view(const Body& b) {
     return k;
 }
 
-// Per-step control block, device resident, always FP64.
+__host__ __device__ inline PlanetKT<float> planet_kernel_view_f(const PlanetK& k) {
+    return {(float)k.m, (float)k.x, (float)k.rs, (float)k.m_over_x2,
+            (float)k.sphi, (float)k.cphi, (float)k.shphi, (float)k.chphi};
+}
+
+// Per-step control block, device resident, FP64; the step's constants also
+// in FP32, so that FP32 kernels read them into scalar registers instead of
+// converting them per cell.
 struct StepCtl {
     double t;            // time at the start of the step
     double dt;           // step size
@@ -81,6 +90,8 @@ struct StepCtl {
     Body planet0;        // planet at t     (first half kick)
     Body planet1;        // planet at t+dt  (predictor and corrector)
     PlanetK pk0, pk1;    // the same, as the source kernel reads them
+    PlanetKT<float> pf0, pf1;   // pk0, pk1
+    float dt_f, h_f;            // dt, dt/2
     double ave_interval; // time-average window (the averaging weight is dt/2 over it)
     double ave_w;        // sum of the averaging weights so far
     int err;             // device loop: 1 once a step found a CFL rate that is not finite and positive

@@ -51,8 +51,8 @@ __device__ __forceinline__ double one_minus_exp_neg(double x) { return -expm1(-x
 // dust does not act back on the gas).  mode 0: the first half kick with the
 // planet at t; 1/2: predictor / corrector with the planet at t+dt, the
 // velocity-dependent forces evaluated at the state predicted over h.
-// h64 = dt/2.  Gas inputs rho, cu, cvp (vp = deviation from vbg), viscous
-// forces Vr, Vp; dust Qu, Qvp.  GAS / DUST select the outputs computed.
+// sv: the step (step_view of that time).  Gas inputs rho, cu, cvp (vp =
+// deviation from vbg), viscous forces Vr, Vp; dust Qu, Qvp.  GAS / DUST select the outputs computed.
 // Used by k_sources and by the x sweeps, which apply the first half kick to
 // the cells they load.
 // The per-radius table values the source terms of one cell read.
@@ -66,17 +66,16 @@ __device__ __forceinline__ SrcTab<real> src_tab(const DiskArgs<real>& d, int ip)
 }
 template <typename real, bool GAS, bool DUST>
 __device__ __forceinline__ void cell_sources(const DiskArgs<real>& d, int mode, const SrcTab<real>& tb, int j,
-                                             double h64, real rho, real cu, real cvp, real Vr, real Vp, real Qu,
-                                             real Qvp, real& nu, real& nvp, real& ndu, real& ndvp) {
-    const real h = (real)h64;
+                                             const StepView<real>& sv, real rho, real cu, real cvp, real Vr, real Vp,
+                                             real Qu, real Qvp, real& nu, real& nvp, real& ndu, real& ndvp) {
+    const real h = sv.h;
     const real mdt = mode == 0 ? real(0) : h;
-    const PlanetK& pk = mode == 0 ? d.ctl->pk0 : d.ctl->pk1;
     const real R = tb.R;
     const real iR = tb.iR;
     const real vbg = tb.vbg;
     const real ebal = tb.ebal;
     real px = real(0), py = real(0);
-    if (d.n_planet > 0) planet_acc(pk, d.phitab + 4 * j, R, px, py);
+    if (d.n_planet > 0) planet_acc(sv.pk, (const PG_CONST real*)d.phitab + 4 * j, R, px, py);
     const real irho = FM<real>::rcp(rho);
     real vx = real(0), vy = real(0);
     if (d.visc) { vx = Vr * irho; vy = Vp * irho; }
@@ -173,7 +172,8 @@ __device__ __forceinline__ void sweep_x_gas_tile(const LaunchSet<real>& ls, int2
     // not ended, and the ended waves free their slots on the CU for other
     // workgroups (the condition is uniform over each wave)
     if ((t & ~63) >= ns) return;
-    const real dt = (real)d.ctl->dt;
+    const StepView<real> sv = step_view<real>(d.ctl, 0);
+    const real dt = sv.dt;
     const PG_GLOBAL real* __restrict__ in = gmem(d.gas[gsel(par)]);
     const size_t row = (size_t)j * nx;
     // The narrow tiles of one slot per thread in every phase (122, 250):
@@ -185,11 +185,12 @@ __device__ __forceinline__ void sweep_x_gas_tile(const LaunchSet<real>& ls, int2
     // uneven disks on 122-radius tiles 321 -> 282 us; the 506-radius tiles
     // of a 1024-radius disk, whose eight waves hide the table loads behind
     // each other, 91 -> 99 us with the 24 more VGPRs, so they load as they go.
+    // (Threads without a slot read the last slot's: 31 registers cleared for
+    // them cost every wave as many instructions.)
     constexpr bool ONE = XBlock<TX>::BT >= XBlock<TX>::S && TX <= 250;
-    real hw[6] = {}, hcs[5] = {}, htp[4] = {}, htr[4] = {}, hgr[2] = {}, hc0[2] = {}, hix[2] = {}, hxa[2] = {};
-    real hixv = real(0), hps = real(0), hir = real(0), hvb = real(0);
-    if (ONE && t < ns - 4) {
-        const int ia = x0 + t + 2;
+    real hw[6], hcs[5], htp[4], htr[4], hgr[2], hc0[2], hix[2], hxa[2], hixv, hps, hir, hvb;
+    if (ONE) {
+        const int ia = min(x0 + t + 2, nx + NPAD);   // threads with no slot read the last one's
         hw[0] = TAB(T_WL0, ia); hw[1] = TAB(T_WL1, ia); hw[2] = TAB(T_WL2, ia);
         hw[3] = TAB(T_WR0, ia); hw[4] = TAB(T_WR1, ia); hw[5] = TAB(T_WR2, ia);
 #pragma unroll
@@ -215,7 +216,7 @@ __device__ __forceinline__ void sweep_x_gas_tile(const LaunchSet<real>& ls, int2
             if (kick) {
                 real Vr = real(0), Vp = real(0), nu, nvp, unused0, unused1;
                 if (d.visc) { Vr = gmem(d.vis)[row + i]; Vp = gmem(d.vis)[N + row + i]; }
-                cell_sources<real, true, false>(d, 0, src_tab(d, ip), j, 0.5 * d.ctl->dt, TAB(T_G_R, ip) + rd, u, vp,
+                cell_sources<real, true, false>(d, 0, src_tab(d, ip), j, sv, TAB(T_G_R, ip) + rd, u, vp,
                                                 Vr, Vp, real(0), real(0), nu, nvp, unused0, unused1);
                 u = nu;
                 vp = nvp;
@@ -248,9 +249,9 @@ __device__ __forceinline__ void sweep_x_gas_tile(const LaunchSet<real>& ls, int2
             tr[m] = ONE ? htr[m] : TAB(T_TBR, ip - 1 + m);
         }
         // differences across the edges ip-1 .. ip+2 (edge e between cells e-1, e)
-        const real p0 = cs[0] * s_r[s - 2], p1 = cs[1] * s_r[s - 1];
-        const real p2 = cs[2] * s_r[s], p3 = cs[3] * s_r[s + 1];
-        const real p4 = cs[4] * s_r[s + 2];
+        const real p0 = mul_rn(cs[0], s_r[s - 2]), p1 = mul_rn(cs[1], s_r[s - 1]);
+        const real p2 = mul_rn(cs[2], s_r[s]), p3 = mul_rn(cs[3], s_r[s + 1]);
+        const real p4 = mul_rn(cs[4], s_r[s + 2]);
         const real dp0 = tp[0] + (p1 - p0), dp1 = tp[1] + (p2 - p1);
         const real dp2 = tp[2] + (p3 - p2), dp3 = tp[3] + (p4 - p3);
         const real r0 = s_r[s - 2], r1 = s_r[s - 1], r2 = s_r[s], r3 = s_r[s + 1], r4 = s_r[s + 2];
@@ -277,13 +278,13 @@ __device__ __forceinline__ void sweep_x_gas_tile(const LaunchSet<real>& ls, int2
         const int ipk = x0 + k;
         const real rbl = ONE ? hgr[0] : TAB(T_G_R, ipk - 1), rbr = ONE ? hgr[1] : TAB(T_G_R, ipk);
         const real cs2l = ONE ? hcs[2] : TAB(T_CS2, ipk - 1), cs2r = ONE ? hcs[3] : TAB(T_CS2, ipk);
-        const real pbl = cs2l * rbl, pbr = cs2r * rbr;
+        const real pbl = mul_rn(cs2l, rbl), pbr = mul_rn(cs2r, rbr);
         real rl, rld, pld, ul, vl, rr, rrd, prd, ur, vr, cl, cr;
-        trace_left_d(ONE ? hc0[0] : TAB(T_C0, ipk - 1), dt, ONE ? hix[0] : TAB(T_IDX, ipk - 1), rbl, pbl, s_r[k - 1], cs2l * s_r[k - 1], s_u[k - 1],
+        trace_left_d(ONE ? hc0[0] : TAB(T_C0, ipk - 1), dt, ONE ? hix[0] : TAB(T_IDX, ipk - 1), rbl, pbl, s_r[k - 1], mul_rn(cs2l, s_r[k - 1]), s_u[k - 1],
                      s_sl[k - 1], s_sr[k - 1], s_sl[S + k - 1], s_sr[S + k - 1],
                      s_sl[2 * S + k - 1], s_sr[2 * S + k - 1],
                      s_sl[3 * S + k - 1], s_L[k - 1], s_sr[3 * S + k - 1], rl, rld, pld, ul, vl, cl);
-        trace_right_d(ONE ? hc0[1] : TAB(T_C0, ipk), dt, ONE ? hix[1] : TAB(T_IDX, ipk), rbr, pbr, s_r[k], cs2r * s_r[k], s_u[k],
+        trace_right_d(ONE ? hc0[1] : TAB(T_C0, ipk), dt, ONE ? hix[1] : TAB(T_IDX, ipk), rbr, pbr, s_r[k], mul_rn(cs2r, s_r[k]), s_u[k],
                       s_sl[k], s_sr[k], s_sl[S + k], s_sr[S + k], s_sl[2 * S + k], s_sr[2 * S + k],
                       s_sl[3 * S + k], s_L[k], s_sr[3 * S + k], rr, rrd, prd, ur, vr, cr);
         real Fr, Fu, FL, presd;
@@ -369,17 +370,17 @@ __device__ __forceinline__ void sweep_x_dust_tile(const LaunchSet<real>& ls, int
     const int nt = min(TX, nx - x0);
     const int ns = nt + 2 * NPAD;
     if ((t & ~63) >= ns) return;   // as in the gas tile
-    const real dt = (real)d.ctl->dt;
+    const StepView<real> sv = step_view<real>(d.ctl, 0);
+    const real dt = sv.dt;
     const PG_GLOBAL real* __restrict__ in = gmem(d.dust[dsel(par)]);
     const size_t row = (size_t)j * nx;
     // the narrow tiles load the table values of the thread's slots here, as
     // the gas tile does (parabola slot ia = x0 + t + 2, interface and update
     // slot ia + 1)
     constexpr bool ONE = XBlock<TX>::BT >= XBlock<TX>::S && TX <= 250;
-    real hw[6] = {}, hix[2] = {};
-    real hxa = real(0), hixv = real(0), hir = real(0), hvb = real(0);
-    if (ONE && t < ns - 4) {
-        const int ia = x0 + t + 2;
+    real hw[6], hix[2], hxa, hixv, hir, hvb;
+    if (ONE) {
+        const int ia = min(x0 + t + 2, nx + NPAD);
         hw[0] = TAB(T_WL0, ia); hw[1] = TAB(T_WL1, ia); hw[2] = TAB(T_WL2, ia);
         hw[3] = TAB(T_WR0, ia); hw[4] = TAB(T_WR1, ia); hw[5] = TAB(T_WR2, ia);
         hix[0] = TAB(T_IDX, ia); hix[1] = TAB(T_IDX, ia + 1);
@@ -398,7 +399,7 @@ __device__ __forceinline__ void sweep_x_dust_tile(const LaunchSet<real>& ls, int
                 const PG_GLOBAL real* __restrict__ g0 = gmem(d.gas[gpre]);
                 const real rho = TAB(T_G_R, ip) + g0[row + i], cu = g0[N + row + i], cvp = g0[2 * N + row + i];
                 real ndu, ndvp, unused0, unused1;
-                cell_sources<real, false, true>(d, 0, src_tab(d, ip), j, 0.5 * d.ctl->dt, rho, cu, cvp, real(0), real(0),
+                cell_sources<real, false, true>(d, 0, src_tab(d, ip), j, sv, rho, cu, cvp, real(0), real(0),
                                                 u, vp, unused0, unused1, ndu, ndvp);
                 u = ndu;
                 vp = ndvp;
@@ -582,7 +583,7 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
     const int ic = live ? i : nx - 1;          // clamped for table reads
     const int ip = ic + NPAD;
     const real iR = TAB(T_IR, ip);
-    const real dt = (real)d.ctl->dt;
+    const real dt = step_view<real>(d.ctl, 0).dt;
     const real dts = dt * iR;                  // set_state / dust_flow receive dt/rad
     const real idy = d.idy;
     const real fup = dt * idy * iR;            // Del.multiply(dt/yv/rad_cyl), sweeps.cu:412
@@ -918,16 +919,15 @@ __global__ __launch_bounds__(256) void k_viscosity(LaunchSet<real> ls, int par, 
 // block instead of a contended atomic on one address.
 template <typename real>
 __device__ __forceinline__ void block_max_store(double* part, real v) {
-    double x = (double)v;
-    for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_xor(x, off, 64));
-    __shared__ double wmax[16];
+    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+    __shared__ real wmax[16];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) wmax[w] = x;
+    if (lane == 0) wmax[w] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
-        double m = 0.0;
+        real m = real(0);
         for (int k = 0; k < (int)((blockDim.x + 63) >> 6); ++k) m = fmax(m, wmax[k]);
-        part[0] = m;
+        part[0] = (double)m;
     }
 }
 
@@ -989,6 +989,7 @@ __global__ __launch_bounds__(256) void k_sources(LaunchSet<real> ls, int par, in
     PG_GLOBAL real* __restrict__ gas = gmem(d.gas[gsel(par)]);
     PG_GLOBAL real* __restrict__ gasT = gmem(d.gas[gsel(par) ^ 1]);
     PG_GLOBAL real* __restrict__ dust = gmem(d.dust[dsel(par)]);
+    const StepView<real> sv = step_view<real>(d.ctl, mode != 0);
     real rate = real(0);
 #pragma unroll
     for (int k = 0; k < TH / PT_TY; ++k) {
@@ -996,7 +997,6 @@ __global__ __launch_bounds__(256) void k_sources(LaunchSet<real> ls, int par, in
         if (i >= nx || j >= ny) break;
         const int ip = i + NPAD;
         const size_t o = (size_t)j * nx + i;
-        const real h = (real)(0.5 * d.ctl->dt);
         const real rd = gas[o], cu = gas[N + o], cvp = gas[2 * N + o];
         const real rho = TAB(T_G_R, ip) + rd;
         real Vr = real(0), Vp = real(0), Qu = real(0), Qvp = real(0);
@@ -1005,16 +1005,16 @@ __global__ __launch_bounds__(256) void k_sources(LaunchSet<real> ls, int par, in
         real nu_ = cu, nvp = cvp, ndu = Qu, ndvp = Qvp;
         if (mode != 3) {
             if (d.has_dust && mode != 1)
-                cell_sources<real, true, true>(d, mode, src_tab(d, ip), j, 0.5 * d.ctl->dt, rho, cu, cvp, Vr, Vp, Qu, Qvp, nu_, nvp, ndu, ndvp);
+                cell_sources<real, true, true>(d, mode, src_tab(d, ip), j, sv, rho, cu, cvp, Vr, Vp, Qu, Qvp, nu_, nvp, ndu, ndvp);
             else
-                cell_sources<real, true, false>(d, mode, src_tab(d, ip), j, 0.5 * d.ctl->dt, rho, cu, cvp, Vr, Vp, Qu, Qvp, nu_, nvp, ndu, ndvp);
+                cell_sources<real, true, false>(d, mode, src_tab(d, ip), j, sv, rho, cu, cvp, Vr, Vp, Qu, Qvp, nu_, nvp, ndu, ndvp);
         }
         real nr_ = rd;   // stored form: the deviation from rho_b
         if (mode == 1) {
             gasT[o] = nr_; gasT[N + o] = nu_; gasT[2 * N + o] = nvp;
         } else {
             if (do_kill) {   // killwave on the corrected state (solve.cu:287-289), toward rho_b
-                const real kk = TAB(T_KILL, ip) * (real)d.ctl->dt;
+                const real kk = TAB(T_KILL, ip) * sv.dt;
                 nr_ += kk * (real(0) - nr_);
                 nu_ += kk * (TAB(T_G_U, ip) - nu_);
                 nvp += kk * (real(0) - nvp);
@@ -1089,6 +1089,7 @@ __global__ __launch_bounds__(256) void k_predvis(LaunchSet<real> ls, int par) {
     const int i0 = (w.y - ty * ntx) * PT_X, j0 = ty * th;
     const PG_GLOBAL real* __restrict__ gas = gmem(d.gas[gsel(par)]);
     const PG_GLOBAL real* __restrict__ vis = gmem(d.vis);
+    const StepView<real> sv = step_view<real>(d.ctl, 1);
     // Slot (lx, ly): radius i = i0 - 1 + lx, row j0 - 1 + ly.  The radius'
     // table values are loaded once per column (a slot past the radial ghost
     // feeds no output and holds the analytic state of radius nx).
@@ -1105,7 +1106,7 @@ __global__ __launch_bounds__(256) void k_predvis(LaunchSet<real> ls, int par) {
             const size_t o = (size_t)j * nx + i;
             const real rho = rb + gas[o], cu = gas[N + o], cvp = gas[2 * N + o];
             real nu_, nvp, unused0, unused1;
-            cell_sources<real, true, false>(d, 1, tb, j, 0.5 * d.ctl->dt, rho, cu, cvp, vis[o], vis[N + o], real(0),
+            cell_sources<real, true, false>(d, 1, tb, j, sv, rho, cu, cvp, vis[o], vis[N + o], real(0),
                                             real(0), nu_, nvp, unused0, unused1);
             r = rho; u = nu_; v = nvp;
         }
@@ -1145,7 +1146,7 @@ __global__ __launch_bounds__(256) void k_predvis(LaunchSet<real> ls, int par) {
                 const size_t o = (size_t)j * nx + i;
                 const real rho = TAB(T_G_R, i + NPAD) + gas[o], cu = gas[N + o], cvp = gas[2 * N + o];
                 real nu_, nvp, unused0, unused1;
-                cell_sources<real, true, false>(d, 1, src_tab(d, i + NPAD), j, 0.5 * d.ctl->dt, rho, cu, cvp, vis[o],
+                cell_sources<real, true, false>(d, 1, src_tab(d, i + NPAD), j, sv, rho, cu, cvp, vis[o],
                                                 vis[N + o], real(0), real(0), nu_, nvp, unused0, unused1);
                 r = rho; u = nu_; v = nvp;
             }
@@ -1192,7 +1193,7 @@ __global__ __launch_bounds__(256) void k_corrvis(LaunchSet<real> ls, int par, in
     PG_GLOBAL real* __restrict__ gasN = gmem(d.gas[gsel(par) ^ 1]);
     PG_GLOBAL real* __restrict__ dust = gmem(d.dust[dsel(par)]);
     const PG_GLOBAL real* __restrict__ vis2 = gmem(d.vis2);
-    const real h = (real)(0.5 * d.ctl->dt);
+    const StepView<real> sv = step_view<real>(d.ctl, 1);
     real rate = real(0);
     // Per-radius table values of a slot column (as in k_predvis).
     struct ColTab {
@@ -1218,14 +1219,14 @@ __global__ __launch_bounds__(256) void k_corrvis(LaunchSet<real> ls, int par, in
             if (d.has_dust) { Qu = dust[N + o]; Qvp = dust[2 * N + o]; }
             real nu_ = cu, nvp = cvp, ndu = Qu, ndvp = Qvp;
             if (d.has_dust)
-                cell_sources<real, true, true>(d, 2, c.src, j, 0.5 * d.ctl->dt, rho, cu, cvp, vis2[o], vis2[N + o], Qu,
+                cell_sources<real, true, true>(d, 2, c.src, j, sv, rho, cu, cvp, vis2[o], vis2[N + o], Qu,
                                                Qvp, nu_, nvp, ndu, ndvp);
             else
-                cell_sources<real, true, false>(d, 2, c.src, j, 0.5 * d.ctl->dt, rho, cu, cvp, vis2[o], vis2[N + o], Qu,
+                cell_sources<real, true, false>(d, 2, c.src, j, sv, rho, cu, cvp, vis2[o], vis2[N + o], Qu,
                                                 Qvp, nu_, nvp, ndu, ndvp);
             real nrd = rd;   // the deviation from rho_b, which wave killing relaxes to 0
             if (do_kill) {
-                const real kk = c.kill * (real)d.ctl->dt;
+                const real kk = c.kill * sv.dt;
                 nrd += kk * (real(0) - nrd);
                 nu_ += kk * (c.gu - nu_);
                 nvp += kk * (real(0) - nvp);
@@ -1450,6 +1451,8 @@ __device__ __forceinline__ void prologue_disk(const DiskArgs<real>& d, int mode,
             if (dts && n0 < d.dts_cap) dts[n0] = dt;
             ctl->nstep = n0 + 1;
         }
+        ctl->dt_f = (float)dt;
+        ctl->h_f = (float)(0.5 * dt);
         s_t = t;
         s_dt = dt;
     }
@@ -1458,8 +1461,8 @@ __device__ __forceinline__ void prologue_disk(const DiskArgs<real>& d, int mode,
     if (tid < 2) {
         orbit_solution(b, tid == 0 ? s_t : s_t + s_dt, d.ramp_time, d.planet_mass, (double)d.frame_omega);
         const PlanetK v = planet_kernel_view(b);
-        if (tid == 0) { ctl->planet0 = b; ctl->pk0 = v; }
-        else { ctl->planet1 = b; ctl->pk1 = v; }
+        if (tid == 0) { ctl->planet0 = b; ctl->pk0 = v; ctl->pf0 = planet_kernel_view_f(v); }
+        else { ctl->planet1 = b; ctl->pk1 = v; ctl->pf1 = planet_kernel_view_f(v); }
     }
     if (oa) {
         const double dt = s_dt;
