@@ -584,8 +584,8 @@ __host__ __device__ inline double ecc_anomaly(double n, double e, double t) {  /
     const double twopi = 2.0 * 3.1415926535897932384626434;
     const double pi = 3.1415926535897932384626434;
     double l = fmod(n * t, twopi);
-    double D = -e * sin(l);
     if (e == 0.0 || l == 0.0 || l == pi || l == twopi) return l;
+    double D = -e * sin(l);
     double step;
     int count = 0;
     do {
@@ -610,8 +610,12 @@ __host__ __device__ inline void orbit_solution(Body& b, double t, double ramp_ti
     double efac = sqrt(1.0 - e * e);
     double B = e / (1.0 + efac);
     double u = ecc_anomaly(n, e, t);
-    double f = u + 2.0 * atan(B * sin(u) / (1.0 - B * cos(u)));
-    double esinf = e * sin(f), ecosf = e * cos(f);
+    double f = u, esinf = 0.0, ecosf = 0.0;   // a circular orbit's anomalies are one
+    if (e != 0.0) {
+        f = u + 2.0 * atan(B * sin(u) / (1.0 - B * cos(u)));
+        esinf = e * sin(f);
+        ecosf = e * cos(f);
+    }
     b.m = ramp_function(t, ramp_time, mass);
     b.x = a * efac * efac / (1.0 + ecosf);
     b.y = f - fmod(frame_omega * t, 2.0 * pi) + pi;
