@@ -313,7 +313,7 @@ struct Group {
     int2* d_wl = nullptr;        // work lists: x sweeps | rings | pointwise kernels
     size_t wl_cap = 0;
     int n_x = 0, n_ring = 0, n_pt = 0;
-    int tile_x = 256, ring_b = RING_THREADS, order = 0;
+    int tile_x = 256, ring_b = RING_TILE, order = 0;
     int pt_rows = PT_YMAX;       // rows of the pointwise/stencil tiles
     bool ave = false;            // time-average the gas around each device-loop step
     int ny_max = 0;
@@ -746,6 +746,23 @@ int auto_pt_rows(const Group& g) {
     return tall >= 1024 ? PT_YMAX : PT_TY;
 }
 
+// Azimuthal tile of a new set of disks: the large one unless the chip holds
+// all its tiles in two rounds (three per CU in FP32, four in FP64): then a
+// pass lasts about as long as two tiles, and smaller ones shorten it by more
+// than their halo costs.  Gas disks, step with 8 x 20 and 8 x 128 tiles:
+// 600x1300 (825 large tiles) 67.5 and 72.2 us, 768x1300 (1056) 75.3 and 78.1,
+// 500x1300 with dust (1386) 76.7 and 78.0, 1024x2048 (2048) 111.8 and 105.7;
+// FP64 with 8 x 20 and 8 x 52: 700x1100 (1936) 108.6 and 110.3, 1024x3072 with
+// dust (15360) 513 and 479.
+int auto_ring(const Group& g) {
+    const int TR = g.prec == 8 ? Launch<double>::phi_tile_radii(RING_TILE) : Launch<float>::phi_tile_radii(RING_TILE);
+    const int TY = g.prec == 8 ? Launch<double>::phi_tile_rows(RING_TILE) : Launch<float>::phi_tile_rows(RING_TILE);
+    long tiles = 0;
+    for (const DiskDev* d : g.disks) tiles += (long)((d->nx + TR - 1) / TR) * ((d->ny + TY - 1) / TY);
+    if (g.dust) tiles *= 2;
+    return tiles <= 2 * 256 * (g.prec == 8 ? 4 : 3) ? 256 : RING_TILE;
+}
+
 int group_schedule(Group& g, int tile_x, int ring_b, int order, int pt_rows) {
     if (!tile_ok(tile_x))
         return fail(PG_E_INVALID, "tile_x=%d: use 122, 128, 250, 256, 384, 506, 512 or 1024", tile_x);
@@ -872,11 +889,11 @@ int group_init(Group& g, int n, const pg_params* params) {
         // 89.3 with 506-cell tiles of eight waves, 80.7 with 250)
         tile = 122;
     }
-    int ringb = RING_THREADS;
+    int ringb = auto_ring(g);
     tile = env_int("PG_TILE_X", tile);
     ringb = env_int("PG_RING_B", ringb);
     if (!tile_ok(tile)) tile = 256;
-    if (!ring_ok(ringb)) ringb = RING_THREADS;
+    if (!ring_ok(ringb)) ringb = auto_ring(g);
     return group_schedule(g, tile, ringb, 0, env_int("PG_PT_ROWS", 0));
 }
 

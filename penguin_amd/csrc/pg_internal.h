@@ -43,7 +43,7 @@ constexpr int PT_X = 64, PT_TY = 4, PT_YMAX = 16;
 constexpr int ADJ_TX = 116;
 constexpr int NGAS = 3;
 constexpr int NDUST = 3;
-constexpr int RING_THREADS = 512;   // default threads per azimuthal-pass block
+constexpr int RING_TILE = 512;   // azimuthal tile of a large disk (PhiTile in pg_kernels.hip)
 
 struct Body {
     double m, a, e, x, y, z, vx, vy, vz, rs;
@@ -203,7 +203,7 @@ struct LaunchSet {
     int tile_x;          // x-sweep tile width (compile-time variants)
     const int2* wl_ring; // rings: local block = radius (-1: padding)
     int n_ring;
-    int ring_b;          // ring chunk (threads per block)
+    int ring_b;          // azimuthal tile (PhiTile)
     int ny_max;          // largest ring, sizes the LDS
     const int2* wl_pt;   // pointwise and stencil kernels: local block = tile tx + ntx * ty
     int n_pt;

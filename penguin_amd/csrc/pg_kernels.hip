@@ -507,19 +507,26 @@ __global__ __launch_bounds__(XBlock<TX>::BT) void k_sweep_x_both(LaunchSet<real>
 }
 
 
-// Tile geometry of the azimuthal pass for a thread count: TR radii x TY
-// output rows.  The rows of one radius are independent of the other radii,
-// so a tile is TR independent azimuthal strips side by side; TR consecutive
-// radii make each row of the tile one contiguous segment in HBM.
-// With 512 threads an FP32 tile is 8 radii x 128 rows (each thread takes two
-// cells of every stage; the 12-row halo is 9 % of the rows swept, against
-// 19 % for 16 x 64 in the same 40 KB of LDS: 73 us against 80 on the
-// 1024x3072 disk; 4 x 256, with 16-byte row segments in HBM, 96 us); an
-// FP64 tile, twice the LDS per cell, 8 x 64.
+// Tile geometry of the azimuthal pass: TR radii x TY output rows by BT
+// threads, named by the schedule's ring_b.  The rows of one radius are
+// independent of the other radii, so a tile is TR independent azimuthal strips
+// side by side; TR consecutive radii make each row of the tile one contiguous
+// segment in HBM.  Every tile sweeps 12 halo rows besides its own.
+//   512: the tile of a large disk.  FP32 8 x 128 (each thread takes two cells
+//        of every stage, the halo is 9 % of the rows swept, 40 KB of LDS;
+//        1024x3072 gas and dust step 199 us, with 8 x 52 by 256 threads 206);
+//        FP64, twice the LDS per cell, 8 x 52 by 256 threads (36 KB, four
+//        tiles per CU: step 479 us, 493 by 512 threads, 520 with 8 x 64).
+//   256: the tile of a disk too small to fill the chip with those: 8 x 20, one
+//        cell per thread and stage, six times the tiles (a 64x128 disk 26.2 us a
+//        step, 29.7 with 8 x 128; 256x512 31.6 against 34.6; 500x1300 48.1
+//        against 52.1), at a halo of 60 % (1024x2048: 111.8 us against 105.7).
 template <typename real, int B> struct PhiTile;
-template <typename real> struct PhiTile<real, 256> { static constexpr int TR = 16, TY = 16; };
-template <typename real> struct PhiTile<real, 512> { static constexpr int TR = 8, TY = sizeof(real) == 4 ? 128 : 64; };
-template <typename real> struct PhiTile<real, 1024> { static constexpr int TR = 16, TY = 64; };
+template <typename real> struct PhiTile<real, 256> { static constexpr int TR = 8, TY = 20, BT = 256; };
+template <typename real> struct PhiTile<real, 512> {
+    static constexpr int TR = 8, TY = sizeof(real) == 4 ? 128 : 52, BT = sizeof(real) == 4 ? 512 : 256;
+};
+template <typename real> struct PhiTile<real, 1024> { static constexpr int TR = 16, TY = 64, BT = 1024; };
 
 // Azimuthal pass of one fluid over a tile, fused with the orbital shift and
 // the residual advection: sweepy_inplace (sweeps.cu:361-456) or
@@ -549,7 +556,7 @@ template <typename real, int B> struct PhiLds {
 };
 template <typename real, bool DUST, int B>
 __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int par, int flags, real* lds) {
-    constexpr int TR = PhiTile<real, B>::TR, TY = PhiTile<real, B>::TY;
+    constexpr int TR = PhiTile<real, B>::TR, TY = PhiTile<real, B>::TY, BT = PhiTile<real, B>::BT;
     constexpr int NK = PhiLds<real, B>::NK;
     constexpr int E = PhiLds<real, B>::E;
     real* const c0 = lds;
@@ -597,15 +604,15 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
     // the sound speed of the radius, read once (the gas interfaces use them)
     const real cs2 = DUST ? real(0) : TAB(T_CS2, ip), cs0 = DUST ? real(0) : TAB(T_C0, ip);
     const real ic0 = DUST ? real(0) : TAB(T_IC0, ip);
-    // B is a multiple of TR, so lane t keeps radius ri in every loop below
-    static_assert(B % TR == 0, "tile");
+    // BT is a multiple of TR, so lane t keeps radius ri in every loop below
+    static_assert(BT % TR == 0, "tile");
 
     // ---- load: TY+12 rows of each radius, shifted back by its inc ----
     const int jbase = y0 - 2 * NPAD - inc;
     const int jb = wrap(jbase + t / TR, ny);   // row of this lane's first element
-    constexpr int KSTEP = B / TR;              // rows advanced per loop trip
+    constexpr int KSTEP = BT / TR;              // rows advanced per loop trip
     int jj = jb;
-    for (int e = t; e < E; e += B) {
+    for (int e = t; e < E; e += BT) {
         real r = DUST ? real(1) : real(0), vp = real(0), u = real(0);
         if (live) {
             const size_t o = (size_t)jj * nx + i;
@@ -619,7 +626,7 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
     }
     __syncthreads();
     // ---- stage A: azimuthal sweep of LDS rows [3, TY+9) ----
-    for (int e = t + 2 * TR; e < (NK - 2) * TR; e += B) {
+    for (int e = t + 2 * TR; e < (NK - 2) * TR; e += BT) {
         const real a0 = c0[e - 2 * TR], a1 = c0[e - TR], a2 = c0[e], a3 = c0[e + TR], a4 = c0[e + 2 * TR];
         const real d0 = a1 - a0, d1 = a2 - a1, d2 = a3 - a2, d3 = a4 - a3;
         // p = c_s^2 rho with c_s^2 fixed along the strip: flatten's
@@ -636,11 +643,11 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
     }
     __syncthreads();
     // interfaces [NPAD, NK-2) of every radius: at most NFA per thread
-    constexpr int FA0 = NPAD * TR, FA1 = (NK - 2) * TR, NFA = (FA1 - FA0 + B - 1) / B;
+    constexpr int FA0 = NPAD * TR, FA1 = (NK - 2) * TR, NFA = (FA1 - FA0 + BT - 1) / BT;
     real fa[NFA][4];
 #pragma unroll
     for (int k = 0; k < NFA; ++k) {
-        const int e = t + FA0 + k * B;
+        const int e = t + FA0 + k * BT;
         if (e >= FA1) break;
         const int m = e - TR;   // the cell left of interface e
         if (DUST) {
@@ -661,13 +668,13 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
     __syncthreads();   // every slope read: the fluxes go over them
 #pragma unroll
     for (int k = 0; k < NFA; ++k) {
-        const int e = t + FA0 + k * B;
+        const int e = t + FA0 + k * BT;
         if (e >= FA1) break;
         F0[e] = fa[k][0]; F1[e] = fa[k][1]; F2[e] = fa[k][2];
         if (!DUST) F3[e] = fa[k][3];
     }
     __syncthreads();
-    for (int e = t + NPAD * TR; e < (NK - NPAD) * TR; e += B) {
+    for (int e = t + NPAD * TR; e < (NK - NPAD) * TR; e += BT) {
         const real Dr = (F0[e] - F0[e + TR]) * fup;
         const real Du = DUST ? (F1[e] - F1[e + TR]) * fup
                              : (F1[e] - F1[e + TR] + (F3[e] - F3[e + TR])) * fup;
@@ -695,13 +702,13 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
         // LDS row k holds swept row y0 - 2 NPAD - inc + k; rows k in
         // [2 NPAD, 2 NPAD + rows) of every tile cover each row once
         PG_GLOBAL real* sw = gmem(d.out_swept);
-        for (int e = t + 2 * NPAD * TR; e < (2 * NPAD + rows) * TR; e += B) {
+        for (int e = t + 2 * NPAD * TR; e < (2 * NPAD + rows) * TR; e += BT) {
             const size_t o = (size_t)wrap(y0 - inc + e / TR - 2 * NPAD, ny) * nx + i;
             sw[o] = c0[e]; sw[N + o] = c2[e]; sw[2 * N + o] = c1[e];
         }
     }
     if (!orbadv) {
-        for (int e = t + 2 * NPAD * TR; e < (2 * NPAD + TY) * TR; e += B) {
+        for (int e = t + 2 * NPAD * TR; e < (2 * NPAD + TY) * TR; e += BT) {
             const int y = e / TR - 2 * NPAD;
             if (!live || y >= rows) continue;
             const size_t o = (size_t)(y0 + y) * nx + i;
@@ -712,7 +719,7 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
     // ---- stage B: residual advection at speed res (advection.cu:1-105) ----
     const real speed = gmem(d.res)[ic];
     const real q = lim01(fabs(speed) * dts * idy);   // |speed| dt / (R dy)
-    for (int e = t + (2 * NPAD - 1) * TR; e < (2 * NPAD + TY + 1) * TR; e += B) {
+    for (int e = t + (2 * NPAD - 1) * TR; e < (2 * NPAD + TY + 1) * TR; e += BT) {
         real l, r;
         slopes(c0[e - 2 * TR], c0[e - TR], c0[e], c0[e + TR], c0[e + 2 * TR], wy[0], wy[1], wy[2], wy[3], wy[4], wy[5], real(0), l, r);
         sl0[e] = l; sr0[e] = r;
@@ -722,11 +729,11 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
         sl2[e] = l; sr2[e] = r;
     }
     __syncthreads();
-    constexpr int FB0 = 2 * NPAD * TR, FB1 = (2 * NPAD + TY + 1) * TR, NFB = (FB1 - FB0 + B - 1) / B;
+    constexpr int FB0 = 2 * NPAD * TR, FB1 = (2 * NPAD + TY + 1) * TR, NFB = (FB1 - FB0 + BT - 1) / BT;
     real fb[NFB][3];
 #pragma unroll
     for (int k = 0; k < NFB; ++k) {
-        const int e = t + FB0 + k * B;
+        const int e = t + FB0 + k * BT;
         if (e >= FB1) break;
         real Dr, Dv, Du;   // Dr: upwind mean of the stored density (gas: its deviation)
         if (speed > real(0)) {
@@ -746,12 +753,12 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
     __syncthreads();   // every slope read: the fluxes go over them
 #pragma unroll
     for (int k = 0; k < NFB; ++k) {
-        const int e = t + FB0 + k * B;
+        const int e = t + FB0 + k * BT;
         if (e >= FB1) break;
         F0[e] = fb[k][0]; F1[e] = fb[k][1]; F2[e] = fb[k][2];
     }
     __syncthreads();
-    for (int e = t + 2 * NPAD * TR; e < (2 * NPAD + TY) * TR; e += B) {
+    for (int e = t + 2 * NPAD * TR; e < (2 * NPAD + TY) * TR; e += BT) {
         const int y = e / TR - 2 * NPAD;
         if (!live || y >= rows) continue;
         const real Dr = (F0[e] - F0[e + TR]) * fup;
@@ -782,12 +789,12 @@ __device__ __forceinline__ void phi_tile(const LaunchSet<real>& ls, int2 w, int 
 // [0, n_ring) the gas tiles, [n_ring, 2 n_ring) the dust tiles; the two
 // fluids read and write different buffers).
 template <typename real, bool DUST, int B>
-__global__ __launch_bounds__(B) void k_phi(LaunchSet<real> ls, int par, int flags) {
+__global__ __launch_bounds__((PhiTile<real, B>::BT)) void k_phi(LaunchSet<real> ls, int par, int flags) {
     __shared__ real lds[PhiLds<real, B>::WORDS];
     phi_tile<real, DUST, B>(ls, ls.wl_ring[blockIdx.x], par, flags, lds);
 }
 template <typename real, int B>
-__global__ __launch_bounds__(B) void k_phi_both(LaunchSet<real> ls, int par, int flags) {
+__global__ __launch_bounds__((PhiTile<real, B>::BT)) void k_phi_both(LaunchSet<real> ls, int par, int flags) {
     __shared__ real lds[PhiLds<real, B>::WORDS];
     const int b = blockIdx.x;
     if (b < ls.n_ring) phi_tile<real, false, B>(ls, ls.wl_ring[b], par, flags, lds);
@@ -1556,11 +1563,11 @@ static hipError_t sweep_x_any(const LaunchSet<real>& ls, int par, int which, int
 template <typename real, int B>
 static hipError_t launch_ring(const LaunchSet<real>& ls, int par, int flags, int which, hipStream_t s) {
     if (which == 1)
-        hipLaunchKernelGGL((k_phi<real, true, B>), dim3(ls.n_ring), dim3(B), 0, s, ls, par, flags);
+        hipLaunchKernelGGL((k_phi<real, true, B>), dim3(ls.n_ring), dim3(PhiTile<real, B>::BT), 0, s, ls, par, flags);
     else if (which == 0)
-        hipLaunchKernelGGL((k_phi<real, false, B>), dim3(ls.n_ring), dim3(B), 0, s, ls, par, flags);
+        hipLaunchKernelGGL((k_phi<real, false, B>), dim3(ls.n_ring), dim3(PhiTile<real, B>::BT), 0, s, ls, par, flags);
     else
-        hipLaunchKernelGGL((k_phi_both<real, B>), dim3(2 * ls.n_ring), dim3(B), 0, s, ls, par, flags);
+        hipLaunchKernelGGL((k_phi_both<real, B>), dim3(2 * ls.n_ring), dim3(PhiTile<real, B>::BT), 0, s, ls, par, flags);
     return hipGetLastError();
 }
 
