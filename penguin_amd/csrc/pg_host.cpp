@@ -877,22 +877,17 @@ int group_init(Group& g, int n, const pg_params* params) {
     const size_t asz = g.prec == 8 ? sizeof(DiskArgs<double>) : sizeof(DiskArgs<float>);
     if ((rc = dev_alloc(g.bytes, &g.d_args, asz * n))) return rc;
     if ((rc = group_upload_args(g))) return rc;
-    // default schedule: widest x tile that divides every disk's radii
-    int tile = 512;
-    for (DiskDev* d : g.disks)
-        if (d->nx % tile) tile = 256;
-    if (n == 1) {
-        // 122-cell tiles: their 128 slots fill two waves, every table value
-        // a thread needs is loaded with the state, and a CU holds up to 16
-        // such workgroups, so one tile's load latency hides behind the
-        // others' arithmetic (the 1024x3072 disk: x sweep 78.5 us against
-        // 89.3 with 506-cell tiles of eight waves, 80.7 with 250)
-        tile = 122;
-    }
+    // default schedule: 122-cell x tiles.  Their 128 slots fill two waves,
+    // every table value a thread needs is loaded with the state, and a CU holds
+    // up to 16 such workgroups, so one tile's load latency hides behind the
+    // others' arithmetic (the 1024x3072 disk: x sweep 78.5 us against 89.3 with
+    // 506-cell tiles of eight waves, 80.7 with 250; 24 disks of 128-512 radii:
+    // step 326 us against 347 with 256-cell tiles, 338 with 250)
+    int tile = 122;
     int ringb = auto_ring(g);
     tile = env_int("PG_TILE_X", tile);
     ringb = env_int("PG_RING_B", ringb);
-    if (!tile_ok(tile)) tile = 256;
+    if (!tile_ok(tile)) tile = 122;
     if (!ring_ok(ringb)) ringb = auto_ring(g);
     return group_schedule(g, tile, ringb, 0, env_int("PG_PT_ROWS", 0));
 }
