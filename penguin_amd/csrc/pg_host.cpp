@@ -1000,9 +1000,9 @@ int vis_start(Group& g) {
     return PG_OK;
 }
 
-int prologue(Group& g, int mode, int do_orbadv) {
-    hipError_t e = g.prec == 8 ? Launch<double>::prologue(g.ls<double>(), mode, do_orbadv, g.stream)
-                               : Launch<float>::prologue(g.ls<float>(), mode, do_orbadv, g.stream);
+int prologue(Group& g, int mode, int do_orbadv, double t = 0.0, double dt = 0.0) {
+    hipError_t e = g.prec == 8 ? Launch<double>::prologue(g.ls<double>(), mode, do_orbadv, g.stream, t, dt)
+                               : Launch<float>::prologue(g.ls<float>(), mode, do_orbadv, g.stream, t, dt);
     if (e != hipSuccess) return fail(PG_E_HIP, "launch prologue failed: %s", hipGetErrorString(e));
     return PG_OK;
 }
@@ -2132,14 +2132,7 @@ int pg_solve(pg_handle* h, double t, double dt) {
     if (h->sph) return pg::sph_solve(h->sph, t, dt);
     Group& g = h->g;
     int rc;
-    if ((rc = pull_ctl(g))) return rc;
-    StepCtl& c = *g.disks[0]->ctl_host;
-    c.t = t;
-    c.dt = dt;
-    c.mode = 0;
-    c.rate_bits = 0ull;
-    if ((rc = push_ctl(g))) return rc;
-    if ((rc = prologue(g, 0, 1))) return rc;
+    if ((rc = prologue(g, 3, 1, t, dt))) return rc;
     if ((rc = passes(g, false))) return rc;
     HIP_TRY(hipStreamSynchronize(g.stream));
     return timers_resolve(g);

@@ -1400,13 +1400,17 @@ __global__ __launch_bounds__(1024) void k_rate_reduce(LaunchSet<real> ls) {
 // sets ctl->err with the step's index and also makes dt 0, so the loop
 // freezes there and the host reports it.
 // mode 2 (replay of a recorded step, one disk): t = td[0], dt = td[1].
+// mode 3 (a step asked for from the host): t and dt are the launch's own, so
+// that no copy of the control block goes either way before the step (256x512
+// disk driven by pg_global_dt and pg_solve: 74 us a step, 59 so).
 // The loads that do not depend on the new step size (the control block, the
 // planets, each thread's first radius of the shift) are issued before the
 // rate reduction, and the two planets (lanes 0 to 3 of wave 0, one evaluation
 // for all) need no barrier before the shifts, which do not read them.
 // The prologue of one disk, by the calling block (any size).
 template <typename real>
-__device__ __forceinline__ void prologue_disk(const DiskArgs<real>& d, int mode, int do_orbadv, const double* td) {
+__device__ __forceinline__ void prologue_disk(const DiskArgs<real>& d, int mode, int do_orbadv, const double* td,
+                                              double2 tv) {
     double* dts = d.dts;
     StepCtl* ctl = d.ctl;
     __shared__ double s_dt, s_t;
@@ -1432,9 +1436,9 @@ __device__ __forceinline__ void prologue_disk(const DiskArgs<real>& d, int mode,
     double rate = mode == 1 ? reduce_partials(d.rate_part, d.rate_nblk) : 0.0;
     if (tid == 0) {
         double t = t0, dt = dt0;
-        if (mode == 2) {
-            t = td[0];
-            dt = td[1];
+        if (mode >= 2) {
+            t = mode == 2 ? td[0] : tv.x;
+            dt = mode == 2 ? td[1] : tv.y;
             ctl->t = t;
             ctl->dt = dt;
         }
@@ -1504,8 +1508,9 @@ __device__ __forceinline__ void prologue_disk(const DiskArgs<real>& d, int mode,
 }
 
 template <typename real>
-__global__ __launch_bounds__(1024) void k_prologue(LaunchSet<real> ls, int mode, int do_orbadv, const double* td) {
-    prologue_disk<real>(ls.disks[blockIdx.x], mode, do_orbadv, td);
+__global__ __launch_bounds__(1024) void k_prologue(LaunchSet<real> ls, int mode, int do_orbadv, const double* td,
+                                                   double2 tv) {
+    prologue_disk<real>(ls.disks[blockIdx.x], mode, do_orbadv, td, tv);
 }
 
 // Replays of n recorded steps at once: block b sets the control block and
@@ -1513,7 +1518,8 @@ __global__ __launch_bounds__(1024) void k_prologue(LaunchSet<real> ls, int mode,
 // (the replays depend on the recorded times only, not on any state).
 template <typename real>
 __global__ __launch_bounds__(1024) void k_prologue_replay(LaunchSet<real> ls, int stride, const double* td) {
-    prologue_disk<real>(ls.disks[(size_t)blockIdx.x * stride], 2, 1, td + 2 * (size_t)blockIdx.x);
+    prologue_disk<real>(ls.disks[(size_t)blockIdx.x * stride], 2, 1, td + 2 * (size_t)blockIdx.x,
+                        double2{0.0, 0.0});
 }
 
 // ------------------------------------------------------------- launchers
@@ -1638,12 +1644,13 @@ struct Launch {
         hipLaunchKernelGGL(k_rate_reduce<real>, dim3(ls.ndisk), dim3(1024), 0, s, ls);
         return hipGetLastError();
     }
-    static hipError_t prologue(const LaunchSet<real>& ls, int mode, int do_orbadv, hipStream_t s) {
-        hipLaunchKernelGGL(k_prologue<real>, dim3(ls.ndisk), dim3(1024), 0, s, ls, mode, do_orbadv, (const double*)nullptr);
+    static hipError_t prologue(const LaunchSet<real>& ls, int mode, int do_orbadv, hipStream_t s, double t, double dt) {
+        hipLaunchKernelGGL(k_prologue<real>, dim3(ls.ndisk), dim3(1024), 0, s, ls, mode, do_orbadv, (const double*)nullptr,
+                           double2{t, dt});
         return hipGetLastError();
     }
     static hipError_t prologue_replay(const LaunchSet<real>& ls, const double* td, hipStream_t s) {
-        hipLaunchKernelGGL(k_prologue<real>, dim3(1), dim3(1024), 0, s, ls, 2, 1, td);
+        hipLaunchKernelGGL(k_prologue<real>, dim3(1), dim3(1024), 0, s, ls, 2, 1, td, double2{0.0, 0.0});
         return hipGetLastError();
     }
     static hipError_t prologue_replay_many(const LaunchSet<real>& ls, int stride, int n, const double* td,

@@ -34,7 +34,9 @@ struct Launch {
     static hipError_t torque(const LaunchSet<real>& ls, int par, double* part, hipStream_t s);
     static hipError_t cfl(const LaunchSet<real>& ls, int par, hipStream_t s);
     static hipError_t rate_reduce(const LaunchSet<real>& ls, hipStream_t s);
-    static hipError_t prologue(const LaunchSet<real>& ls, int mode, int do_orbadv, hipStream_t s);
+    // t, dt: the step's in mode 3
+    static hipError_t prologue(const LaunchSet<real>& ls, int mode, int do_orbadv, hipStream_t s, double t = 0.0,
+                               double dt = 0.0);
     // replay of a recorded step: t = td[0], dt = td[1] (one disk)
     static hipError_t prologue_replay(const LaunchSet<real>& ls, const double* td, hipStream_t s);
     // n replays: descriptor b * stride of ls.disks from t = td[2b], dt = td[2b+1]
