@@ -701,14 +701,19 @@ __global__ __launch_bounds__(AdjPhiTile<real>::TR * AdjPhiTile<real>::TY) void k
 
 // ------------------------------------------------------ viscosity adjoint
 // Forward: k_viscosity / vis_from_tile, a 9-point stencil of (rho nu, u, vp).
-// Per output cell, the adjoints it sends to each input of its stencil:
-// lu[n], lv[n] for the u and vp of neighbour n, ln[n] for its rho nu
-// (nonzero for n = 0, 1, 2, 4, 7); neighbour n = 3b + a at radius i-1+a,
-// row j, j-1, j+1 for b = 0, 1, 2.  Returns X fx + Y fy (the forces are
-// linear in nu, hence in alpha).
+// Each coefficient of the stencil belongs to the output's radius, and an
+// output sends its neighbours only 12 different numbers (AV_*): what it sends
+// to a side neighbour, and one per field for the four corners, whose signs
+// alternate.  What it sends to its own inputs goes to self (u, vp, rho nu).
+// Row neighbours are named by the side of the output they lie on.  Returns
+// X fx + Y fy (the forces are linear in nu, hence in alpha).
+enum { AV_U_IN, AV_U_OUT, AV_U_DN, AV_U_UP, AV_U_X, AV_V_IN, AV_V_OUT, AV_V_DN, AV_V_UP, AV_V_X, AV_N_R, AV_N_P, AV_N };
+
+// neighbour n = 3b + a of the output at radius i, row j is radius i-1+a, row
+// j, j-1, j+1 for b = 0, 1, 2
 template <typename real>
 __device__ __forceinline__ double vis_adj_cell(const DiskArgs<real>& d, int ip, const real* nr, const real* u,
-                                               const real* v, real X, real Y, real* lu, real* lv, real* ln) {
+                                               const real* v, real X, real Y, real* o, real* self) {
     const real i20 = TAB(T_I20, ip), i21 = TAB(T_I21, ip), i10 = TAB(T_I10, ip);
     const real ir = TAB(T_IR, ip), idy = d.idy, hdy = real(0.5) * idy;
     const real dudx = (u[2] - u[0]) * i20;
@@ -738,44 +743,35 @@ __device__ __forceinline__ double vis_adj_cell(const DiskArgs<real>& d, int ip, 
               real(2) * sxy * ir;
         lal = (double)X * (double)fx + (double)Y * (double)fy;
     }
-    // adjoints of the derivative terms
-    const real l_dndx = X * (real(2) * dudx) + Y * ((dudy + dvdx) - v1 * ir);
-    const real l_dudx = X * (real(2) * dndx + real(2) * n1 * ir);
-    const real l_n1 = X * (real(2) * d2udx2 + real(2) * dudx * ir + (d2udy2 + d2vdxy) - dvdy * ir -
-                           real(2) * (dvdy + u[1] * ir) * ir) +
-                      Y * (real(2) * d2vdy2 + real(2) * dudy * ir + (d2udxy + d2vdx2) - dvdx * ir + v1 * ir * ir +
-                           real(2) * (dudy + dvdx - v1 * ir) * ir);
-    const real l_d2udx2 = X * real(2) * n1;
-    const real l_dndy = X * ((dudy + dvdx) - v1 * ir) + Y * (real(2) * dvdy + real(2) * u[1] * ir);
-    const real l_dudy = X * dndy + Y * (real(4) * n1 * ir + dndx);
-    const real l_dvdx = X * dndy + Y * (dndx + n1 * ir);
-    const real l_d2udy2 = X * n1, l_d2vdxy = X * n1;
-    const real l_v1 = X * (-dndy * ir) + Y * (-dndx * ir - n1 * ir * ir);
-    const real l_dvdy = X * (real(-3) * n1 * ir) + Y * (real(2) * dndy);
-    const real l_u1 = X * (real(-2) * n1 * ir * ir) + Y * (real(2) * dndy * ir);
-    const real l_d2vdy2 = Y * real(2) * n1, l_d2udxy = Y * n1, l_d2vdx2 = Y * n1;
-    for (int n = 0; n < 9; ++n) { lu[n] = real(0); lv[n] = real(0); ln[n] = real(0); }
-    lu[2] += l_dudx * i20; lu[0] -= l_dudx * i20;
-    {
-        const real c = real(2) * i20 * l_d2udx2;
-        lu[2] += c * i21; lu[1] -= c * (i21 + i10); lu[0] += c * i10;
-    }
-    lv[2] += l_dvdx * i20; lv[0] -= l_dvdx * i20;
-    {
-        const real c = real(2) * i20 * l_d2vdx2;
-        lv[2] += c * i21; lv[1] -= c * (i21 + i10); lv[0] += c * i10;
-    }
-    ln[2] += l_dndx * i20; ln[0] -= l_dndx * i20;
-    lv[7] += l_dvdy * ky; lv[4] -= l_dvdy * ky;
-    lv[7] += l_d2vdy2 * kyy; lv[1] -= real(2) * l_d2vdy2 * kyy; lv[4] += l_d2vdy2 * kyy;
-    lv[8] += l_d2vdxy * kxy; lv[6] -= l_d2vdxy * kxy; lv[5] -= l_d2vdxy * kxy; lv[3] += l_d2vdxy * kxy;
-    lu[7] += l_dudy * ky; lu[4] -= l_dudy * ky;
-    lu[7] += l_d2udy2 * kyy; lu[1] -= real(2) * l_d2udy2 * kyy; lu[4] += l_d2udy2 * kyy;
-    lu[8] += l_d2udxy * kxy; lu[6] -= l_d2udxy * kxy; lu[5] -= l_d2udxy * kxy; lu[3] += l_d2udxy * kxy;
-    ln[7] += l_dndy * ky; ln[4] -= l_dndy * ky;
-    lv[1] += l_v1;
-    ln[1] += l_n1;
-    lu[1] += l_u1;
+    // adjoints of the derivative terms, times the terms' coefficients
+    const real shear = (dudy + dvdx) - v1 * ir;
+    const real n_r = (X * (real(2) * dudx) + Y * shear) * i20;                              // dndx
+    const real n_p = (X * shear + Y * (real(2) * dvdy + real(2) * u[1] * ir)) * ky;         // dndy
+    const real u_r = X * (real(2) * dndx + real(2) * n1 * ir) * i20;                        // dudx
+    const real u_p = (X * dndy + Y * (real(4) * n1 * ir + dndx)) * ky;                      // dudy
+    const real v_r = (X * dndy + Y * (dndx + n1 * ir)) * i20;                               // dvdx
+    const real v_p = (X * (real(-3) * n1 * ir) + Y * (real(2) * dndy)) * ky;                // dvdy
+    const real Xn = X * n1, Yn = Y * n1;
+    const real u_rr = real(4) * i20 * Xn, u_pp = Xn * kyy;                                  // d2udx2, d2udy2
+    const real v_rr = real(2) * i20 * Yn, v_pp = real(2) * Yn * kyy;                        // d2vdx2, d2vdy2
+    o[AV_U_IN] = u_rr * i10 - u_r;
+    o[AV_U_OUT] = u_rr * i21 + u_r;
+    o[AV_U_DN] = u_pp - u_p;
+    o[AV_U_UP] = u_pp + u_p;
+    o[AV_U_X] = Yn * kxy;                                                                   // d2udxy
+    o[AV_V_IN] = v_rr * i10 - v_r;
+    o[AV_V_OUT] = v_rr * i21 + v_r;
+    o[AV_V_DN] = v_pp - v_p;
+    o[AV_V_UP] = v_pp + v_p;
+    o[AV_V_X] = Xn * kxy;                                                                   // d2vdxy
+    o[AV_N_R] = n_r;
+    o[AV_N_P] = n_p;
+    self[0] = X * (real(-2) * n1 * ir * ir) + Y * (real(2) * dndy * ir) - u_rr * (i21 + i10) - real(2) * u_pp;
+    self[1] = X * (-dndy * ir) + Y * (-dndx * ir - n1 * ir * ir) - v_rr * (i21 + i10) - real(2) * v_pp;
+    self[2] = X * (real(2) * d2udx2 + real(2) * dudx * ir + (d2udy2 + d2vdxy) - dvdy * ir -
+                   real(2) * (dvdy + u[1] * ir) * ir) +
+              Y * (real(2) * d2vdy2 + real(2) * dudy * ir + (d2udxy + d2vdx2) - dvdx * ir + v1 * ir * ir +
+                   real(2) * shear * ir);
     return lal;
 }
 
@@ -791,10 +787,11 @@ template <typename real>
 __device__ __forceinline__ void src_adj_cell(const DiskArgs<real>& d, int mode, int ip, int j, real h, real rho,
                                              real cvp, real Vr, real Vp, real lnr, real lnu, real lnv, real& lrho,
                                              real& lu, real& lcvp, real& lVr, real& lVp, double& lq) {
-    const PlanetK& pk = mode == 0 ? d.ctl->pk0 : d.ctl->pk1;
+    const PG_CONST StepCtl* ctl = (const PG_CONST StepCtl*)d.ctl;
+    const PG_CONST PlanetK* pk = mode == 0 ? &ctl->pk0 : &ctl->pk1;
     const real iR = TAB(T_IR, ip), vbg = TAB(T_VBG, ip);
     real px = real(0), py = real(0);
-    if (d.n_planet > 0) planet_acc(pk, (const PG_CONST real*)d.phitab + 4 * j, TAB(T_XC, ip), px, py);
+    if (d.n_planet > 0) planet_acc(*pk, (const PG_CONST real*)d.phitab + 4 * j, TAB(T_XC, ip), px, py);
     const real irho = FM<real>::rcp(rho);
     if (!d.visc) { Vr = real(0); Vp = real(0); }
     const real vy = Vp * irho;
@@ -818,9 +815,14 @@ __device__ __forceinline__ void src_adj_cell(const DiskArgs<real>& d, int mode, 
 
 // Viscosity adjoint on tiles of AV_X radii x TH rows, fused with the
 // pointwise passes around it.  The outputs whose stencil meets the tile
-// (the tile and a one-cell halo) compute their partial adjoints into LDS
-// from the forward state staged with a two-cell halo; each tile cell then
-// gathers what its 3x3 neighbours sent.
+// (the tile and a one-cell halo) put the 12 numbers that they send their
+// neighbours into LDS, from the forward state staged with a two-cell halo;
+// each tile cell then gathers what its 3x3 neighbours sent.  A thread
+// computes the output at its own cell first, so what a cell sends to itself
+// and what the source pass there sends to the state stay in registers.
+// Latency between the barriers bounds it, so waves per SIMD count: with each
+// output's 23 stencil adjoints in LDS one block of 8 waves filled a CU's LDS
+// in FP64 (512x1024: modes 1 and 2 56 and 46 us, now 44 and 35).
 //   MODE 0: V = vis(S): lvis -> li (module entry point).
 //   MODE 1: end of the step: corrector S4 = C(S3, V1) (lo = adjoint of S4,
 //           s = S3, vis = V1), V1 = vis(T) (s2 = T), predictor
@@ -831,12 +833,12 @@ __device__ __forceinline__ void src_adj_cell(const DiskArgs<real>& d, int mode, 
 constexpr int AV_X = 64;
 
 template <typename real, int MODE, int TH>
-__global__ __launch_bounds__(AV_X * TH) void k_adj_vis(AdjArgs<real> A) {
+__global__ __launch_bounds__(AV_X * TH, 4) void k_adj_vis(AdjArgs<real> A) {
     constexpr int B = AV_X * TH;
     constexpr int H1X = AV_X + 2, H1 = H1X * (TH + 2);   // outputs: tile + 1
     constexpr int H2X = AV_X + 4, H2 = H2X * (TH + 4);   // their state: tile + 2
     __shared__ real sr[H2], su[H2], sv[H2];
-    __shared__ real P[23][H1];
+    __shared__ real P[AV_N][H1];
     const DiskArgs<real>& d = *A.d;
     const int nx = d.nx, ny = d.ny;
     const size_t N = (size_t)nx * ny;
@@ -859,104 +861,99 @@ __global__ __launch_bounds__(AV_X * TH) void k_adj_vis(AdjArgs<real> A) {
     }
     __syncthreads();
     double lal = 0.0, lq = 0.0;
+    real own[3] = {real(0), real(0), real(0)};   // sent by this cell's output to itself: u, vp, rho nu
+    real src[3] = {real(0), real(0), real(0)};   // sent by this cell's source pass to rho, u, vp
+    // outputs: the B cells of the tile, then its halo (the two rows beside
+    // it, then the columns)
     for (int e = t; e < H1; e += B) {
-        const int lx = e % H1X, ly = e / H1X;
+        int lx, ly;
+        if (e < B) {
+            lx = e % AV_X + 1; ly = e / AV_X + 1;
+        } else if (e < B + 2 * H1X) {
+            lx = (e - B) % H1X; ly = e - B < H1X ? 0 : TH + 1;
+        } else {
+            const int k = e - B - 2 * H1X;
+            lx = k & 1 ? AV_X + 1 : 0; ly = (k >> 1) + 1;
+        }
         const int i = i0 - 1 + lx, jr = j0 - 1 + ly, j = wrap(jr, ny);
-        real lu[9], lv[9], ln[9];
-        for (int n = 0; n < 9; ++n) { lu[n] = real(0); lv[n] = real(0); ln[n] = real(0); }
-        real nu[3] = {real(0), real(0), real(0)};
+        real out[AV_N];
+        for (int n = 0; n < AV_N; ++n) out[n] = real(0);
         if (i >= 0 && i < nx) {
             const int ip = i + NPAD;
             const size_t o = (size_t)j * nx + i;
-            real X, Y;
-            double lq_unused = 0.0;
+            real X, Y, a[3], self[3];
+            double lqc = 0.0;
             if (MODE == 0) {
                 X = A.lvis[o]; Y = A.lvis[N + o];
             } else {
                 // adjoint of the forces from the source pass that read them
-                real a0, a1, a2;
                 src_adj_cell(d, MODE == 1 ? 2 : 0, ip, j, h, TAB(T_G_R, ip) + A.s[o], A.s[2 * N + o], A.vis[o], A.vis[N + o], A.lo[o],
-                             A.lo[N + o], A.lo[2 * N + o], a0, a1, a2, X, Y, lq_unused);
+                             A.lo[N + o], A.lo[2 * N + o], a[0], a[1], a[2], X, Y, lqc);
                 if (MODE == 2) { X += A.lvis[o]; Y += A.lvis[N + o]; }
             }
-            for (int n = 0; n < 3; ++n) nu[n] = TAB(T_NU, ip - 1 + n);
             real nr[9], u[9], v[9];
             const int rows[3] = {ly + 1, ly, ly + 2};   // H2 rows of j, j-1, j+1
 #pragma unroll
             for (int b = 0; b < 3; ++b)
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const int n = 3 * b + a, s = rows[b] * H2X + lx + a;
-                    nr[n] = sr[s] * nu[a]; u[n] = su[s]; v[n] = sv[s];
+                for (int c = 0; c < 3; ++c) {
+                    const int n = 3 * b + c, s = rows[b] * H2X + lx + c;
+                    nr[n] = sr[s] * TAB(T_NU, ip - 1 + c); u[n] = su[s]; v[n] = sv[s];
                 }
-            const double l = vis_adj_cell(d, ip, nr, u, v, X, Y, lu, lv, ln);
-            if (lx >= 1 && lx <= AV_X && ly >= 1 && ly <= TH && jr < ny) lal += l;   // each output once
+            const double l = vis_adj_cell(d, ip, nr, u, v, X, Y, out, self);
+            if (e < B && jr < ny) {   // each output once
+                lal += l;
+                lq += lqc;
+                for (int n = 0; n < 3; ++n) {
+                    own[n] = self[n];
+                    if (MODE != 0) src[n] = a[n];
+                }
+            }
         }
-        for (int n = 0; n < 9; ++n) { P[n][e] = lu[n]; P[9 + n][e] = lv[n]; }
-        P[18][e] = ln[0] * nu[0]; P[19][e] = ln[1] * nu[1]; P[20][e] = ln[2] * nu[2];
-        P[21][e] = ln[4] * nu[1]; P[22][e] = ln[7] * nu[1];
+        for (int n = 0; n < AV_N; ++n) P[n][ly * H1X + lx] = out[n];
     }
     __syncthreads();
-    // what the outputs sent to the cell at H1 slot (cx, cy): output
-    // (cx + 1 - a, cy - db) holds it as its neighbour n = 3b + a
-    // (slots outside the H1 columns hold no output: skipped for the ghost
-    // columns, whose outer neighbours are not radii of the disk)
-    auto gather = [&](int cx, int cy, real& gr, real& gu, real& gv) {
-        gr = gu = gv = real(0);
-        const int db[3] = {0, -1, 1};
-#pragma unroll
-        for (int b = 0; b < 3; ++b)
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const int ox = cx + 1 - a;
-                if (ox < 0 || ox >= H1X) continue;
-                const int n = 3 * b + a, e = (cy - db[b]) * H1X + ox;
-                gu += P[n][e];
-                gv += P[9 + n][e];
-                if (n == 0) gr += P[18][e];
-                else if (n == 1) gr += P[19][e];
-                else if (n == 2) gr += P[20][e];
-                else if (n == 4) gr += P[21][e];
-                else if (n == 7) gr += P[22][e];
-            }
-    };
     const int cx = t % AV_X + 1, cy = t / AV_X + 1;
     const int i = i0 + cx - 1, j = j0 + cy - 1;
+    // what the outputs around H1 slot c sent it: the output at c + 1 holds it
+    // as its inner neighbour, the one at c - 1 as its outer, the one at
+    // c + H1X as the row below it, the one at c - H1X as the row above
+    const int c = cy * H1X + cx;
     if (j < ny) {
         // radial ghost columns next to this cell: their u = -1.5 nu/R is
-        // proportional to alpha
+        // proportional to alpha (only this column of outputs is beside them)
         if (i == 0) {
-            real gr, gu, gv;
-            gather(cx - 1, cy, gr, gu, gv);
+            const real gu = P[AV_U_IN][c] + (P[AV_U_X][c + H1X] - P[AV_U_X][c - H1X]);
             lal += (double)gu * (double)TAB(T_G_U, -1 + NPAD);
         }
         if (i == nx - 1) {
-            real gr, gu, gv;
-            gather(cx + 1, cy, gr, gu, gv);
+            const real gu = P[AV_U_OUT][c] + (P[AV_U_X][c - H1X] - P[AV_U_X][c + H1X]);
             lal += (double)gu * (double)TAB(T_G_U, nx + NPAD);
         }
         if (i < nx) {
             const int ip = i + NPAD;
             const size_t o = (size_t)j * nx + i;
-            real gr, gu, gv;
-            gather(cx, cy, gr, gu, gv);
+            auto corners = [&](const real* p) {
+                return (p[c - H1X - 1] - p[c - H1X + 1]) + (p[c + H1X + 1] - p[c + H1X - 1]);
+            };
+            const real gu = own[0] + (P[AV_U_IN][c + 1] + P[AV_U_OUT][c - 1]) +
+                            (P[AV_U_DN][c + H1X] + P[AV_U_UP][c - H1X]) + corners(P[AV_U_X]);
+            const real gv = own[1] + (P[AV_V_IN][c + 1] + P[AV_V_OUT][c - 1]) +
+                            (P[AV_V_DN][c + H1X] + P[AV_V_UP][c - H1X]) + corners(P[AV_V_X]);
+            const real gr = TAB(T_NU, ip) * (own[2] + (P[AV_N_R][c - 1] - P[AV_N_R][c + 1]) +
+                                             (P[AV_N_P][c - H1X] - P[AV_N_P][c + H1X]));
             if (MODE == 0) {
                 put(A.li, o, gr, A.accumulate & 1);
                 put(A.li, N + o, gu, A.accumulate & 1);
                 put(A.li, 2 * N + o, gv, A.accumulate & 1);
             } else if (MODE == 1) {
-                real cr, cu, cv, cX, cY, pr, pu, pv, pX, pY;
-                src_adj_cell(d, 2, ip, j, h, TAB(T_G_R, ip) + A.s[o], A.s[2 * N + o], A.vis[o], A.vis[N + o], A.lo[o], A.lo[N + o],
-                             A.lo[2 * N + o], cr, cu, cv, cX, cY, lq);
+                real pr, pu, pv, pX, pY;
                 src_adj_cell(d, 1, ip, j, h, TAB(T_G_R, ip) + A.s[o], A.s[2 * N + o], A.vis2[o], A.vis2[N + o], gr, gu, gv, pr, pu, pv,
                              pX, pY, lq);
-                A.li[o] = cr + pr; A.li[N + o] = cu + pu; A.li[2 * N + o] = cv + pv;
+                A.li[o] = src[0] + pr; A.li[N + o] = src[1] + pu; A.li[2 * N + o] = src[2] + pv;
                 A.lvis[o] = pX; A.lvis[N + o] = pY;
             } else {
-                real kr, ku, kv, kX, kY;
-                src_adj_cell(d, 0, ip, j, h, TAB(T_G_R, ip) + A.s[o], A.s[2 * N + o], A.vis[o], A.vis[N + o], A.lo[o], A.lo[N + o],
-                             A.lo[2 * N + o], kr, ku, kv, kX, kY, lq);
-                A.li[o] = kr + gr; A.li[N + o] = ku + gu; A.li[2 * N + o] = kv + gv;
+                A.li[o] = src[0] + gr; A.li[N + o] = src[1] + gu; A.li[2 * N + o] = src[2] + gv;
             }
         }
     }
@@ -1017,8 +1014,9 @@ struct AdjLaunch {
         hipLaunchKernelGGL(k_adj_adv<real>, dim3((nx + TR - 1) / TR, (ny + TY - 1) / TY), dim3(TR * TY), 0, s, A);
         return hipGetLastError();
     }
-    // viscosity tiles: 64 x 8 (two blocks per CU in FP32)
-    static constexpr int THV = 8;
+    // viscosity tiles: 64 x 7 in FP64, two blocks to the LDS of a CU (75 KB;
+    // 83 KB and one block with 8 rows)
+    static constexpr int THV = sizeof(real) == 8 ? 7 : 8;
     // mode 0: viscosity alone; 1: corrector + viscosity + predictor;
     // 2: kick + viscosity (AdjArgs field use: k_adj_vis)
     static hipError_t vis(const AdjArgs<real>& A, int mode, int nx, int ny, hipStream_t s) {

@@ -1444,15 +1444,14 @@ struct AdjWork {
 
 namespace {
 
-// workgroups of the largest adjoint grid (x adjoint: 256-radius tiles x
-// rows; source adjoints: 256-radius segments x rows; azimuthal adjoints:
-// 8-radius x 16-row tiles at most; viscosity: 64 x 8 tiles at most)
+// workgroups of the largest adjoint grid that sums a parameter adjoint (x
+// adjoint: ADJ_TX-radius tiles x rows; source adjoints: 256-radius segments x
+// rows; viscosity: 64 x 7 tiles, the smaller ones of FP64)
 int adj_slots(int nx, int ny) {
     const int a = ((nx + ADJ_TX - 1) / ADJ_TX) * ny;   // x-sweep adjoint tiles
     const int b = ((nx + 2 + 255) / 256) * ny;
-    const int c = ((nx + 7) / 8) * ((ny + 15) / 16);
-    const int v = ((nx + 63) / 64) * ((ny + 7) / 8);   // viscosity tiles (the smaller, FP64)
-    return std::max(std::max(a, v), std::max(b, c));
+    const int v = ((nx + 63) / 64) * ((ny + 6) / 7);
+    return std::max(a, std::max(b, v));
 }
 
 void adj_free(AdjWork* w) {
