@@ -303,17 +303,21 @@ __global__ __launch_bounds__(AdjXBlock<TX>::B) void k_adj_x(AdjArgs<real> A) {
 
 // ------------------------------------------------- azimuthal sweep adjoint
 // Tile of TR radii x TY output rows, no shift (the pass SA = sweep(S2));
-// LDS row k <-> row y0-6+k, rows [0, TY+12).
-// FP32: 16 radii x 32 rows, 512 threads, two cells per thread (the 12-row
-// halo adds 38 % to the rows swept, against 75 % for 16-row tiles); FP64
-// 8 x 16 within the LDS of a CU.
-template <typename real> struct AdjPhiTile {
-    static constexpr int TR = sizeof(real) == 8 ? 8 : 16, TY = sizeof(real) == 8 ? 16 : 32;
+// LDS row k <-> row y0-6+k, rows [0, TY+12).  BT threads, two cells each.
+// Arithmetic on the tile and its 12-row halo bounds these kernels, at the two
+// or three waves per SIMD that their registers allow, so the tiles are as tall
+// as two (azimuthal) and three (advection) blocks in a CU's LDS leave them.
+// FP64 512x1024, against 8 x 16 tiles by 128 threads: azimuthal 97.8 -> 59.7
+// us, advection 30.5 -> 24.9.
+template <typename real, int TY_> struct AdjTile {
+    static constexpr int TR = sizeof(real) == 8 ? 8 : 16, TY = TY_, BT = sizeof(real) == 8 ? 256 : 512;
 };
+template <typename real> using AdjPhiTile = AdjTile<real, 46>;
+template <typename real> using AdjAdvTile = AdjTile<real, 44>;
 
 template <typename real>
-__global__ __launch_bounds__(AdjPhiTile<real>::TR * AdjPhiTile<real>::TY) void k_adj_phi(AdjArgs<real> A) {
-    constexpr int TR = AdjPhiTile<real>::TR, TY = AdjPhiTile<real>::TY, B = TR * TY;
+__global__ __launch_bounds__(AdjPhiTile<real>::BT) void k_adj_phi(AdjArgs<real> A) {
+    constexpr int TR = AdjPhiTile<real>::TR, TY = AdjPhiTile<real>::TY, B = AdjPhiTile<real>::BT;
     constexpr int NK = TY + 4 * NPAD, E = NK * TR;
     constexpr int NT = (E + B - 1) / B;   // cells per thread
     __shared__ real c0[E], c1[E], c2[E], fl[E];
@@ -322,9 +326,10 @@ __global__ __launch_bounds__(AdjPhiTile<real>::TR * AdjPhiTile<real>::TY) void k
     // (1) of the parabola reversal
     __shared__ real W[13][E];
     // per-interface adjoints sent to the left cell (those sent to the right
-    // cell stay in the registers of the thread that owns it); CL[0..4] then
-    // hold the flattening adjoints of the pressures
-    __shared__ real CL[TC_N][E];
+    // cell stay in the registers of the thread that owns it), the first four
+    // over the fluxes, which the update's reversal has consumed; the last five
+    // then hold the flattening adjoints of the pressures
+    __shared__ real CLx[TC_N - 4][E];
     real (*sl)[E] = W;
     real (*sr)[E] = W + 3;
     real *F0 = W[6], *F1 = W[7], *F2 = W[8], *F3 = W[9];
@@ -448,11 +453,20 @@ __global__ __launch_bounds__(AdjPhiTile<real>::TR * AdjPhiTile<real>::TY) void k
             trace_left_c_adj(cs0, ic0, dts, idy, inL, lSc[0], lSc[1], lSc[2], lL);
             trace_right_c_adj(cs0, ic0, dts, idy, inR, lSc[3], lSc[4], lSc[5], lR[q]);
         }
-        for (int m = 0; m < TC_N; ++m) CL[m][e] = lL[m];
+        for (int m = 0; m < TC_N; ++m) (m < 4 ? W[6 + m] : CLx[m - 4])[e] = lL[m];
     }
     __syncthreads();
     // gather per cell (right cell of interface k, left cell of interface
-    // k+1), then the reverse of its parabolas: adjoints of the neighbour
+    // k+1)
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+        const int e = t + q * B;
+        const int k = e / TR;
+        if (e < E && k + 1 >= NPAD && k + 1 <= NK - 3)
+            for (int m = 0; m < TC_N; ++m) lR[q][m] += (m < 4 ? W[6 + m] : CLx[m - 4])[e + TR];
+    }
+    __syncthreads();
+    // then the reverse of its parabolas: adjoints of the neighbour
     // differences and of the flattening coefficient (into W)
     real (*ld)[4][E] = reinterpret_cast<real (*)[4][E]>(&W[0][0]);
     real* lfl = W[12];
@@ -461,10 +475,7 @@ __global__ __launch_bounds__(AdjPhiTile<real>::TR * AdjPhiTile<real>::TY) void k
         const int e = t + q * B;
         if (e >= E) break;
         const int k = e / TR;
-        real g[TC_N];
-        for (int m = 0; m < TC_N; ++m) g[m] = lR[q][m];   // zero unless interface e exists
-        if (k + 1 >= NPAD && k + 1 <= NK - 3)
-            for (int m = 0; m < TC_N; ++m) g[m] += CL[m][e + TR];
+        const real* g = lR[q];   // zero where no interface is
         a0[q] += g[TC_R]; a1[q] += g[TC_U]; a2[q] += g[TC_V];
         const real asl[3] = {g[TC_RSL], g[TC_USL], g[TC_VSL]}, asr[3] = {g[TC_RSR], g[TC_USR], g[TC_VSR]};
         real lflat = real(0);
@@ -485,7 +496,7 @@ __global__ __launch_bounds__(AdjPhiTile<real>::TR * AdjPhiTile<real>::TY) void k
         lfl[e] = lflat;
     }
     __syncthreads();
-    real (*lfp)[E] = CL;
+    real (*lfp)[E] = CLx;
 #pragma unroll
     for (int q = 0; q < NT; ++q) {
         const int e = t + q * B;
@@ -529,8 +540,8 @@ __global__ __launch_bounds__(AdjPhiTile<real>::TR * AdjPhiTile<real>::TY) void k
 // takes pre-shift row y - inc.  Tile of TR radii x TY pre-shift rows y0..;
 // LDS row k <-> pre-shift row y0-6+k <-> post-shift row y0-6+k+inc.
 template <typename real>
-__global__ __launch_bounds__(AdjPhiTile<real>::TR * AdjPhiTile<real>::TY) void k_adj_adv(AdjArgs<real> A) {
-    constexpr int TR = AdjPhiTile<real>::TR, TY = AdjPhiTile<real>::TY, B = TR * TY;
+__global__ __launch_bounds__(AdjAdvTile<real>::BT) void k_adj_adv(AdjArgs<real> A) {
+    constexpr int TR = AdjAdvTile<real>::TR, TY = AdjAdvTile<real>::TY, B = AdjAdvTile<real>::BT;
     constexpr int NK = TY + 4 * NPAD, E = NK * TR;
     constexpr int NT = (E + B - 1) / B;   // cells per thread
     __shared__ real c0[E], c1[E], c2[E];
@@ -1005,13 +1016,15 @@ struct AdjLaunch {
         return hipGetLastError();
     }
     static hipError_t phi(const AdjArgs<real>& A, int nx, int ny, hipStream_t s) {
-        constexpr int TR = AdjPhiTile<real>::TR, TY = AdjPhiTile<real>::TY;
-        hipLaunchKernelGGL(k_adj_phi<real>, dim3((nx + TR - 1) / TR, (ny + TY - 1) / TY), dim3(TR * TY), 0, s, A);
+        using Tile = AdjPhiTile<real>;
+        constexpr int TR = Tile::TR, TY = Tile::TY;
+        hipLaunchKernelGGL(k_adj_phi<real>, dim3((nx + TR - 1) / TR, (ny + TY - 1) / TY), dim3(Tile::BT), 0, s, A);
         return hipGetLastError();
     }
     static hipError_t adv(const AdjArgs<real>& A, int nx, int ny, hipStream_t s) {
-        constexpr int TR = AdjPhiTile<real>::TR, TY = AdjPhiTile<real>::TY;
-        hipLaunchKernelGGL(k_adj_adv<real>, dim3((nx + TR - 1) / TR, (ny + TY - 1) / TY), dim3(TR * TY), 0, s, A);
+        using Tile = AdjAdvTile<real>;
+        constexpr int TR = Tile::TR, TY = Tile::TY;
+        hipLaunchKernelGGL(k_adj_adv<real>, dim3((nx + TR - 1) / TR, (ny + TY - 1) / TY), dim3(Tile::BT), 0, s, A);
         return hipGetLastError();
     }
     // viscosity tiles: 64 x 7 in FP64, two blocks to the LDS of a CU (75 KB;
