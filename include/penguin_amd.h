@@ -245,8 +245,8 @@ int pg_batch_run(pg_batch* b, int nsteps, double* t_io, double* dt_io, double* d
 /* launch schedule: x-sweep tile width (128, 256, 384, 512, 1024, or 122,
    250, 506, whose tiles with their 6 halo cells fill 2, 4, 8 waves);
    azimuthal tile (256: 8 radii x 20 rows, 512: 8 x 128, FP64 8 x 52, 1024: 16 x 64);
-   azimuthal tile order (0: each XCD a contiguous band of tile rows of every
-   disk, 1: row by row, 2: radius strip by strip); rows of the pointwise and
+   azimuthal tile order (0: each XCD a contiguous eighth of the tiles of all
+   disks, 1: row by row, 2: radius strip by strip); rows of the pointwise and
    stencil tiles (4, 8 or 16; 0 = chosen from the batch size) */
 int pg_batch_set_schedule(pg_batch* b, int tile_x, int ring_b, int order, int pt_rows);
 int pg_batch_get_schedule(pg_batch* b, int* tile_x, int* ring_b, int* order, int* pt_rows);

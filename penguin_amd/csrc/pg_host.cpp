@@ -668,43 +668,42 @@ int disk_create(const pg_params& P, hipStream_t s, DiskDev** out) {
 // ------------------------------------------------------------ groups
 // Work lists of one launch schedule.
 //   x sweeps: every (tile, row) of every disk, disk by disk; pointwise and
-//   stencil kernels: every PT_X x pt_rows tile, tile rows in
-//   XCD-contiguous bands.
-//   azimuthal pass: tiles of TR radii x TY rows (tile = ty * ntr + tr).
+//   stencil kernels: every PT_X x pt_rows tile; azimuthal pass: tiles of TR
+//   radii x TY rows (tile = ty * ntr + tr).
 //   Workgroups are dispatched round-robin over the 8 XCDs, each with its own
-//   L2.  Tiles that are neighbours in azimuth share their 6-row halos and
-//   tiles that are neighbours in radius share cache lines, so with order 0
-//   each disk's tile rows are cut into 8 contiguous runs and XCD x receives
-//   run x (entry 8k+x of the list), radius strips innermost.  Order 1 lists
-//   the tiles row by row, order 2 strip by strip.  Entries with tile -1 pad
-//   the list.
+//   L2.  Tiles that are neighbours in azimuth share their halo rows and tiles
+//   that are neighbours in radius share cache lines, so the pointwise tiles,
+//   and with order 0 the azimuthal ones, are cut into 8 contiguous runs of the
+//   list of all disks' tiles, row by row, and XCD x receives run x (entry
+//   8k+x).  Runs differ by one tile at most: cut disk by disk into runs of
+//   whole tile rows, a 1300-row ring's eleven rows of tiles went two to an XCD
+//   and none to the last two, and the rings of a batch, of 2 to 12 rows of
+//   tiles each, mostly to the first XCDs (24 disks' azimuthal pass 123 us, 90
+//   now; the 600x1300 disk's step with these tiles 72.2 us, 62.7 now).  Order
+//   1 lists the azimuthal tiles row by row, order 2 strip by strip.  Entries
+//   with tile -1 pad the list.
+void deal_xcds(const std::vector<int2>& tiles, std::vector<int2>& out) {
+    const size_t n = tiles.size(), len = (n + 7) / 8;
+    out.assign(8 * len, make_int2(0, -1));
+    for (size_t x = 0; x < 8; ++x)
+        for (size_t k = x * n / 8, e = (x + 1) * n / 8, slot = 0; k < e; ++k, ++slot) out[8 * slot + x] = tiles[k];
+}
+
 void build_worklists(const Group& g, int tile_x, int ring_b, int order, int pt_rows, std::vector<int2>& wx,
                      std::vector<int2>& wr, std::vector<int2>& wp) {
     wx.clear();
     wr.clear();
     wp.clear();
     const int nd = g.ndisk();
-    // pointwise kernels (the viscosity stencil reads rows j-1, j, j+1): each
-    // XCD receives a contiguous band of rows of every disk, so neighbouring
-    // rows are read through one L2
-    std::vector<int2> qp[8];
+    std::vector<int2> tiles;
     for (int k = 0; k < nd; ++k) {
         const DiskDev* d = g.disks[k];
-        const int tiles = (d->nx + tile_x - 1) / tile_x;
-        for (int b = 0; b < tiles * d->ny; ++b) wx.push_back(make_int2(k, b));
+        const int ntx_x = (d->nx + tile_x - 1) / tile_x;
+        for (int b = 0; b < ntx_x * d->ny; ++b) wx.push_back(make_int2(k, b));
         const int ntx = (d->nx + PT_X - 1) / PT_X, nty = (d->ny + pt_rows - 1) / pt_rows;
-        const int per = (nty + 7) / 8;
-        for (int x = 0; x < 8; ++x)
-            for (int ty = x * per; ty < std::min((x + 1) * per, nty); ++ty)
-                for (int tx = 0; tx < ntx; ++tx) qp[x].push_back(make_int2(k, tx + ntx * ty));
+        for (int b = 0; b < ntx * nty; ++b) tiles.push_back(make_int2(k, b));
     }
-    {
-        size_t len = 0;
-        for (int x = 0; x < 8; ++x) len = std::max(len, qp[x].size());
-        wp.assign(8 * len, make_int2(0, -1));
-        for (int x = 0; x < 8; ++x)
-            for (size_t k = 0; k < qp[x].size(); ++k) wp[8 * k + x] = qp[x][k];
-    }
+    deal_xcds(tiles, wp);
     const int TR = g.prec == 8 ? Launch<double>::phi_tile_radii(ring_b) : Launch<float>::phi_tile_radii(ring_b);
     const int TY = g.prec == 8 ? Launch<double>::phi_tile_rows(ring_b) : Launch<float>::phi_tile_rows(ring_b);
     if (order != 0) {
@@ -719,19 +718,12 @@ void build_worklists(const Group& g, int tile_x, int ring_b, int order, int pt_r
         }
         return;
     }
-    std::vector<int2> q[8];
+    tiles.clear();
     for (int k = 0; k < nd; ++k) {
         const int ntr = (g.disks[k]->nx + TR - 1) / TR, nty = (g.disks[k]->ny + TY - 1) / TY;
-        const int per = (nty + 7) / 8;
-        for (int x = 0; x < 8; ++x)
-            for (int ty = x * per; ty < std::min((x + 1) * per, nty); ++ty)
-                for (int tr = 0; tr < ntr; ++tr) q[x].push_back(make_int2(k, ty * ntr + tr));
+        for (int b = 0; b < ntr * nty; ++b) tiles.push_back(make_int2(k, b));
     }
-    size_t len = 0;
-    for (int x = 0; x < 8; ++x) len = std::max(len, q[x].size());
-    wr.assign(8 * len, make_int2(0, -1));
-    for (int x = 0; x < 8; ++x)
-        for (size_t k = 0; k < q[x].size(); ++k) wr[8 * k + x] = q[x][k];
+    deal_xcds(tiles, wr);
 }
 
 bool tile_ok(int t) {
@@ -752,21 +744,22 @@ int auto_pt_rows(const Group& g) {
     return tall >= 1024 ? PT_YMAX : PT_TY;
 }
 
-// Azimuthal tile of a new set of disks: the large one unless the chip holds
-// all its tiles in two rounds (three per CU in FP32, four in FP64): then a
-// pass lasts about as long as two tiles, and smaller ones shorten it by more
-// than their halo costs.  Gas disks, step with 8 x 20 and 8 x 128 tiles:
-// 600x1300 (825 large tiles) 67.5 and 72.2 us, 768x1300 (1056) 75.3 and 78.1,
-// 500x1300 with dust (1386) 76.7 and 78.0, 1024x2048 (2048) 111.8 and 105.7;
-// FP64 with 8 x 20 and 8 x 52: 700x1100 (1936) 108.6 and 110.3, 1024x3072 with
-// dust (15360) 513 and 479.
+// Azimuthal tile of a new set of disks: the large one unless there are fewer
+// than 4.5 of them per CU, about what a CU holds at a time: then a pass lasts
+// as long as one or two tiles, and smaller ones shorten it by more than their
+// halo costs.  Step with 8 x 20 and 8 x 128 tiles, us: 256x512 (128 large
+// tiles) 26.5 and 29.4, 600x1300 (825) 61.4 and 62.7, 768x1300 (1056) 69.6 and
+// 71.0, six disks (1280) 80.9 and 78.8, 500x1300 with dust (1386) 70.2 and
+// 68.9, 1024x2048 (2048) 109.4 and 103.5; FP64 with 8 x 20 and 8 x 52: 600x700
+// (1050) 69.8 and 71.0, 333x777 with dust (1260) 68.8 and 68.5, 700x1100 (1936)
+// 101.8 and 101.7, 1024x2048 (5120) 203.6 and 197.6.
 int auto_ring(const Group& g) {
     const int TR = g.prec == 8 ? Launch<double>::phi_tile_radii(RING_TILE) : Launch<float>::phi_tile_radii(RING_TILE);
     const int TY = g.prec == 8 ? Launch<double>::phi_tile_rows(RING_TILE) : Launch<float>::phi_tile_rows(RING_TILE);
     long tiles = 0;
     for (const DiskDev* d : g.disks) tiles += (long)((d->nx + TR - 1) / TR) * ((d->ny + TY - 1) / TY);
     if (g.dust) tiles *= 2;
-    return tiles <= 2 * 256 * (g.prec == 8 ? 4 : 3) ? 256 : RING_TILE;
+    return 2 * tiles <= 9 * 256 ? 256 : RING_TILE;
 }
 
 int group_schedule(Group& g, int tile_x, int ring_b, int order, int pt_rows) {
