@@ -69,10 +69,9 @@ template <> struct FM<double> {
 };
 
 // ---------------------------------------------------------------- helpers
-// A product that is rounded before it is added to anything: where a sum of two
-// products could contract either into a fused multiply-add, the choice would
-// be the compiler's in each tile variant, and the variants' results would
-// differ in the last bit.
+// A product that is rounded before it is added to anything, where the compiler
+// could otherwise contract it into a fused multiply-add in one kernel and not in
+// another.
 template <typename real>
 PG_HD real mul_rn(real a, real b) {
 #pragma clang fp contract(off)
@@ -640,17 +639,17 @@ template <typename real, typename PK>
 __device__ __forceinline__ void planet_acc(const PK& pk, const PG_CONST real* pt, real R, real& ax, real& ay) {
     const real sp = (real)pk.sphi, cp = (real)pk.cphi, shp = (real)pk.shphi, chp = (real)pk.chphi;
     // sums of two products in a written order, so that every kernel variant
-    // rounds them alike (see mul_rn)
+    // rounds them alike
     const real s = fma(pt[0], cp, -(pt[1] * sp));      // sin(phi - phi_p)
-    const real c = fma(pt[1], cp, pt[0] * sp);         // cos(phi - phi_p)
+    const real c = fma(pt[0], sp, pt[1] * cp);         // cos(phi - phi_p)
     const real h = fma(pt[2], chp, -(pt[3] * shp));    // sin((phi - phi_p)/2)
     const real px = (real)pk.x, m = (real)pk.m, rs = (real)pk.rs;
-    const real Rp2 = fma(R - px, R - px, fma(real(4) * px * R * h, h, rs * rs));
+    const real Rp2 = fma(rs, rs, fma(R - px, R - px, real(4) * px * R * h * h));
     const real iRp = FM<real>::rsqrt(Rp2);
     const real k = iRp * iRp * iRp;
     const real ind = (real)pk.m_over_x2;
     ax = fma(-m * fma(-px, c, R), k, -(c * ind));
-    ay = fma(-m * px * s, k, s * ind);
+    ay = fma(s, ind, -(m * px * s * k));
 }
 
 // What the source terms read of the step, in the storage precision: dt, dt/2

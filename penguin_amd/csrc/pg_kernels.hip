@@ -64,7 +64,10 @@ template <typename real>
 __device__ __forceinline__ SrcTab<real> src_tab(const DiskArgs<real>& d, int ip) {
     return {TAB(T_XC, ip), TAB(T_IR, ip), TAB(T_VBG, ip), TAB(T_EBAL, ip), TAB(T_TS, ip), TAB(T_ITS, ip)};
 }
-template <typename real, bool GAS, bool DUST>
+// RN: the gas's radial kick is rounded before it is added (the corrector and
+// the module entry point in FP32) instead of fused into the sum: written out,
+// so that the result does not depend on where the compiler puts that sum.
+template <typename real, bool GAS, bool DUST, bool RN = false>
 __device__ __forceinline__ void cell_sources(const DiskArgs<real>& d, int mode, const SrcTab<real>& tb, int j,
                                              const StepView<real>& sv, real rho, real cu, real cvp, real Vr, real Vp,
                                              real Qu, real Qvp, real& nu, real& nvp, real& ndu, real& ndvp) {
@@ -100,7 +103,7 @@ __device__ __forceinline__ void cell_sources(const DiskArgs<real>& d, int mode, 
         }
     }
     if (GAS) {
-        nu = cu + axg(Tvp) * h;
+        nu = RN ? cu + mul_rn(axg(Tvp), h) : cu + axg(Tvp) * h;
         nvp = cvp + ay * h;
     }
     if (DUST) {
@@ -249,9 +252,9 @@ __device__ __forceinline__ void sweep_x_gas_tile(const LaunchSet<real>& ls, int2
             tr[m] = ONE ? htr[m] : TAB(T_TBR, ip - 1 + m);
         }
         // differences across the edges ip-1 .. ip+2 (edge e between cells e-1, e)
-        const real p0 = mul_rn(cs[0], s_r[s - 2]), p1 = mul_rn(cs[1], s_r[s - 1]);
-        const real p2 = mul_rn(cs[2], s_r[s]), p3 = mul_rn(cs[3], s_r[s + 1]);
-        const real p4 = mul_rn(cs[4], s_r[s + 2]);
+        const real p0 = cs[0] * s_r[s - 2], p1 = cs[1] * s_r[s - 1];
+        const real p2 = cs[2] * s_r[s], p3 = cs[3] * s_r[s + 1];
+        const real p4 = cs[4] * s_r[s + 2];
         const real dp0 = tp[0] + (p1 - p0), dp1 = tp[1] + (p2 - p1);
         const real dp2 = tp[2] + (p3 - p2), dp3 = tp[3] + (p4 - p3);
         const real r0 = s_r[s - 2], r1 = s_r[s - 1], r2 = s_r[s], r3 = s_r[s + 1], r4 = s_r[s + 2];
@@ -278,13 +281,13 @@ __device__ __forceinline__ void sweep_x_gas_tile(const LaunchSet<real>& ls, int2
         const int ipk = x0 + k;
         const real rbl = ONE ? hgr[0] : TAB(T_G_R, ipk - 1), rbr = ONE ? hgr[1] : TAB(T_G_R, ipk);
         const real cs2l = ONE ? hcs[2] : TAB(T_CS2, ipk - 1), cs2r = ONE ? hcs[3] : TAB(T_CS2, ipk);
-        const real pbl = mul_rn(cs2l, rbl), pbr = mul_rn(cs2r, rbr);
+        const real pbl = cs2l * rbl, pbr = cs2r * rbr;
         real rl, rld, pld, ul, vl, rr, rrd, prd, ur, vr, cl, cr;
-        trace_left_d(ONE ? hc0[0] : TAB(T_C0, ipk - 1), dt, ONE ? hix[0] : TAB(T_IDX, ipk - 1), rbl, pbl, s_r[k - 1], mul_rn(cs2l, s_r[k - 1]), s_u[k - 1],
+        trace_left_d(ONE ? hc0[0] : TAB(T_C0, ipk - 1), dt, ONE ? hix[0] : TAB(T_IDX, ipk - 1), rbl, pbl, s_r[k - 1], cs2l * s_r[k - 1], s_u[k - 1],
                      s_sl[k - 1], s_sr[k - 1], s_sl[S + k - 1], s_sr[S + k - 1],
                      s_sl[2 * S + k - 1], s_sr[2 * S + k - 1],
                      s_sl[3 * S + k - 1], s_L[k - 1], s_sr[3 * S + k - 1], rl, rld, pld, ul, vl, cl);
-        trace_right_d(ONE ? hc0[1] : TAB(T_C0, ipk), dt, ONE ? hix[1] : TAB(T_IDX, ipk), rbr, pbr, s_r[k], mul_rn(cs2r, s_r[k]), s_u[k],
+        trace_right_d(ONE ? hc0[1] : TAB(T_C0, ipk), dt, ONE ? hix[1] : TAB(T_IDX, ipk), rbr, pbr, s_r[k], cs2r * s_r[k], s_u[k],
                       s_sl[k], s_sr[k], s_sl[S + k], s_sr[S + k], s_sl[2 * S + k], s_sr[2 * S + k],
                       s_sl[3 * S + k], s_L[k], s_sr[3 * S + k], rr, rrd, prd, ur, vr, cr);
         real Fr, Fu, FL, presd;
@@ -518,9 +521,9 @@ __global__ __launch_bounds__(XBlock<TX>::BT) void k_sweep_x_both(LaunchSet<real>
 //        FP64, twice the LDS per cell, 8 x 52 by 256 threads (36 KB, four
 //        tiles per CU: step 479 us, 493 by 512 threads, 520 with 8 x 64).
 //   256: the tile of a disk too small to fill the chip with those: 8 x 20, one
-//        cell per thread and stage, six times the tiles (a 64x128 disk 26.2 us a
-//        step, 29.7 with 8 x 128; 256x512 31.6 against 34.6; 500x1300 48.1
-//        against 52.1), at a halo of 60 % (1024x2048: 111.8 us against 105.7).
+//        cell per thread and stage, six times the tiles (a 256x512 gas disk's
+//        step 26.5 us, 29.4 with 8 x 128; 400x1000 42.3 against 43.5), at a halo
+//        of 60 % (1024x2048: 109.4 us against 103.5).
 template <typename real, int B> struct PhiTile;
 template <typename real> struct PhiTile<real, 256> { static constexpr int TR = 8, TY = 20, BT = 256; };
 template <typename real> struct PhiTile<real, 512> {
@@ -1014,9 +1017,9 @@ __global__ __launch_bounds__(256) void k_sources(LaunchSet<real> ls, int par, in
         real nu_ = cu, nvp = cvp, ndu = Qu, ndvp = Qvp;
         if (mode != 3) {
             if (d.has_dust && mode != 1)
-                cell_sources<real, true, true>(d, mode, src_tab(d, ip), j, sv, rho, cu, cvp, Vr, Vp, Qu, Qvp, nu_, nvp, ndu, ndvp);
+                cell_sources<real, true, true, sizeof(real) == 4>(d, mode, src_tab(d, ip), j, sv, rho, cu, cvp, Vr, Vp, Qu, Qvp, nu_, nvp, ndu, ndvp);
             else
-                cell_sources<real, true, false>(d, mode, src_tab(d, ip), j, sv, rho, cu, cvp, Vr, Vp, Qu, Qvp, nu_, nvp, ndu, ndvp);
+                cell_sources<real, true, false, sizeof(real) == 4>(d, mode, src_tab(d, ip), j, sv, rho, cu, cvp, Vr, Vp, Qu, Qvp, nu_, nvp, ndu, ndvp);
         }
         real nr_ = rd;   // stored form: the deviation from rho_b
         if (mode == 1) {
@@ -1228,10 +1231,10 @@ __global__ __launch_bounds__(256) void k_corrvis(LaunchSet<real> ls, int par, in
             if (d.has_dust) { Qu = dust[N + o]; Qvp = dust[2 * N + o]; }
             real nu_ = cu, nvp = cvp, ndu = Qu, ndvp = Qvp;
             if (d.has_dust)
-                cell_sources<real, true, true>(d, 2, c.src, j, sv, rho, cu, cvp, vis2[o], vis2[N + o], Qu,
+                cell_sources<real, true, true, sizeof(real) == 4>(d, 2, c.src, j, sv, rho, cu, cvp, vis2[o], vis2[N + o], Qu,
                                                Qvp, nu_, nvp, ndu, ndvp);
             else
-                cell_sources<real, true, false>(d, 2, c.src, j, sv, rho, cu, cvp, vis2[o], vis2[N + o], Qu,
+                cell_sources<real, true, false, sizeof(real) == 4>(d, 2, c.src, j, sv, rho, cu, cvp, vis2[o], vis2[N + o], Qu,
                                                 Qvp, nu_, nvp, ndu, ndvp);
             real nrd = rd;   // the deviation from rho_b, which wave killing relaxes to 0
             if (do_kill) {
