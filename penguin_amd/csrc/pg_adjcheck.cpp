@@ -85,4 +85,9 @@ int adjc_eval(int fn, const double* x, const double* ly, double* y, double* lx) 
     return 0;
 }
 
+// slopes in FP32: x as fn 2 takes it
+void adjc_slopes_f32(const float* x, float* y) {
+    slopes(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7], x[8], x[9], x[10], x[11], y[0], y[1]);
+}
+
 }  // extern "C"

@@ -69,6 +69,18 @@ template <> struct FM<double> {
 };
 
 // ---------------------------------------------------------------- helpers
+// A minimum of two and a zero that together keep a value which is not a number:
+// in FP32 by the minimum itself, one instruction like the one that drops it
+// (v_minimum3_f32); FP64 has none, so there the zero is x - x.
+template <typename real> struct MinNan;
+template <> struct MinNan<float> {
+    static PG_HD float min(float a, float b) { return __builtin_elementwise_minimum(a, b); }
+    static PG_HD float zero(float) { return 0.0f; }
+};
+template <> struct MinNan<double> {
+    static PG_HD double min(double a, double b) { return fmin(a, b); }
+    static PG_HD double zero(double x) { return x - x; }
+};
 // A product that is rounded before it is added to anything, where the compiler
 // could otherwise contract it into a fused multiply-add in one kernel and not in
 // another.
@@ -104,12 +116,15 @@ PG_HD void slopes_d(real d0, real d1, real d2, real d3,
     // The common factor fk carries the sign of d1 and the zero.  (With the
     // conditions as branches every sweep was 2-3 % slower: the 1024x3072 gas and
     // dust step 228 us against 222, in FP64 567 against 552.)
+    // A difference that is not a number makes both slopes so (it would be lost
+    // in the minima, and the zero factor hides it).
     real l = fmin(fabs(wl0 * d0 + wl1 * d1 + wl2 * d2), fabs(d1));
     real r = fmin(fabs(wr0 * d1 + wr1 * d2 + wr2 * d3), fabs(d2));
-    const real fk = copysign(d1 * d2 > real(0) ? real(1) - flat : real(0), d1);
+    const real d12 = d1 * d2;
+    const real fk = copysign(d12 > real(0) ? real(1) - flat : MinNan<real>::zero(d12), d1);
     const real l2 = l + l, r2 = r + r;
-    l = fk * fmin(l, r2);
-    r = fk * fmin(r, l2);
+    l = fk * MinNan<real>::min(l, r2);
+    r = fk * MinNan<real>::min(r, l2);
     sL = l;
     sR = r;
 }
