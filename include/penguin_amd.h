@@ -86,7 +86,8 @@ int pg_solve(pg_handle* h, double t, double dt);
    the 1.1x cap, clipped to end_time) entirely on the device; t and dt live
    in device memory.  *t_io / *dt_io carry the time and the previous step in
    and out; dts (nsteps doubles, may be NULL) receives every step size.
-   use_graph != 0 captures one step in a hipGraph and replays it. */
+   use_graph != 0 captures steps in hipGraphs, of 16, 4 and 1 steps as the run
+   needs them, and replays them; they are kept for later runs. */
 int pg_run(pg_handle* h, int nsteps, double* t_io, double* dt_io, double* dts, int use_graph);
 
 /* ---- module-level entry points (reference module boundaries) ---------- */

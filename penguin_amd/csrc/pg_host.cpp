@@ -1054,6 +1054,59 @@ int group_stage(Group& g, size_t bytes) {
     return PG_OK;
 }
 
+// The longest graph that the steps left fill.
+int graph_level(int left) {
+    int level = 0;
+    while (GRAPH_STEPS[level] > left) ++level;
+    return level;
+}
+
+// The graph of GRAPH_STEPS[level] steps from the present parity, captured if
+// it is not there yet; the host's parity bookkeeping advances as if they had
+// run (a capture records the steps without running them).
+int graph_next_steps(Group& g, int level, hipGraphExec_t* out) {
+    const int p0 = g.par(), p = p0 | (level << 2);
+    if (!g.graph[p]) {
+        hipGraph_t gr = nullptr;
+        HIP_TRY(hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal));
+        int rc = PG_OK;
+        for (int k = 0; k < GRAPH_STEPS[level] && !rc; ++k) {
+            rc = prologue(g, 1, 1);
+            if (!rc) rc = average_pass(g);
+            if (!rc) rc = passes(g, true);
+            if (!rc) rc = average_pass(g);
+        }
+        hipError_t ec = hipStreamEndCapture(g.stream, &gr);
+        if (!rc && ec != hipSuccess) rc = fail(PG_E_HIP, "hipStreamEndCapture: %s", hipGetErrorString(ec));
+        if (!rc && (ec = hipGraphInstantiate(&g.graph[p], gr, nullptr, nullptr, 0)) != hipSuccess) {
+            g.graph[p] = nullptr;
+            rc = fail(PG_E_HIP, "hipGraphInstantiate: %s", hipGetErrorString(ec));
+        }
+        if (gr) (void)hipGraphDestroy(gr);
+        if (rc) {
+            g.set_par(p0);
+            return rc;
+        }
+        g.graph_next[p] = g.par();
+    }
+    g.set_par(g.graph_next[p]);
+    *out = g.graph[p];
+    return PG_OK;
+}
+
+// Every graph that a run of nsteps replays, captured beforehand, so that none
+// is recorded and instantiated (about 20 us for each step in it) while a run
+// is being timed on the device.
+int graphs_ready(Group& g, int nsteps) {
+    const int p0 = g.par();
+    int rc = PG_OK;
+    hipGraphExec_t x;
+    for (int n = 0, level; n < nsteps && !rc; n += GRAPH_STEPS[level])
+        rc = graph_next_steps(g, level = graph_level(nsteps - n), &x);
+    g.set_par(p0);
+    return rc;
+}
+
 // nsteps of the reference loop (main.cu:320-359) for every disk of the
 // group, each with its own dt.  t_io/dt_io hold one entry per disk; dts
 // (ndisk*nsteps, disk-major, may be null) receives the step sizes;
@@ -1092,40 +1145,17 @@ int group_run(Group& g, int nsteps, double* t_io, double* dt_io, double* dts, in
     // the corrector), and its viscous forces
     if ((rc = launch_cfl(g))) return rc;
     if ((rc = vis_start(g))) return rc;
-    if (loop_ms) HIP_TRY(hipEventRecord(g.ev_a, g.stream));
+    if (loop_ms) {
+        if (use_graph && !g.profile && (rc = graphs_ready(g, nsteps))) return rc;
+        HIP_TRY(hipEventRecord(g.ev_a, g.stream));
+    }
     if (use_graph && !g.profile) {
         for (int n = 0; n < nsteps;) {
-            // the longest graph that the steps left fill
-            int level = 0;
-            while (GRAPH_STEPS[level] > nsteps - n) ++level;
-            const int len = GRAPH_STEPS[level], p = g.par() | (level << 2);
-            if (!g.graph[p]) {
-                // capture records the steps without running them; the host's
-                // parity bookkeeping advances as if they had run
-                hipGraph_t gr;
-                HIP_TRY(hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal));
-                int rc2 = PG_OK;
-                for (int k = 0; k < len && !rc2; ++k) {
-                    rc2 = prologue(g, 1, 1);
-                    if (!rc2) rc2 = average_pass(g);
-                    if (!rc2) rc2 = passes(g, true);
-                    if (!rc2) rc2 = average_pass(g);
-                }
-                hipError_t ec = hipStreamEndCapture(g.stream, &gr);
-                if (rc2) return rc2;
-                if (ec != hipSuccess) return fail(PG_E_HIP, "hipStreamEndCapture: %s", hipGetErrorString(ec));
-                ec = hipGraphInstantiate(&g.graph[p], gr, nullptr, nullptr, 0);
-                (void)hipGraphDestroy(gr);
-                if (ec != hipSuccess) {
-                    g.graph[p] = nullptr;
-                    return fail(PG_E_HIP, "hipGraphInstantiate: %s", hipGetErrorString(ec));
-                }
-                g.graph_next[p] = g.par();
-            } else {
-                g.set_par(g.graph_next[p]);
-            }
-            HIP_TRY(hipGraphLaunch(g.graph[p], g.stream));
-            n += len;
+            const int level = graph_level(nsteps - n);
+            hipGraphExec_t x;
+            if ((rc = graph_next_steps(g, level, &x))) return rc;
+            HIP_TRY(hipGraphLaunch(x, g.stream));
+            n += GRAPH_STEPS[level];
         }
     } else {
         for (int n = 0; n < nsteps; ++n) {
@@ -1322,7 +1352,8 @@ int group_autotune(Group& g, int steps, double* best_ms) {
             t[k] = saved_ctl[k].t;
             dt[k] = saved_ctl[k].dt > 0.0 ? saved_ctl[k].dt : g.disks[k]->P.end_time;
         }
-        // first call captures the graph and warms up; the second is timed
+        // the first call warms up; the second is timed, its graphs captured
+        // before the time is taken
         if ((r = group_run(g, 1, t.data(), dt.data(), nullptr, 1, nullptr)) ||
             (r = group_run(g, n, t.data(), dt.data(), nullptr, 1, &ms)) || (r = restore()))
             return r;
