@@ -13,7 +13,8 @@ time loop does it.
 
 Prints one JSON line.  `value` is interior cell updates per second over the
 K timed steps (state resident in HBM before timing starts; the device loop
-replays its captured step).  `roofline` describes the dominant kernel:
+replays captured steps: a graph longer than the warm-up's steps needed, up to
+16 steps, is captured by the timed run itself, about 20 us a step in it).  `roofline` describes the dominant kernel:
 algorithmic bytes per launch over its average duration from HIP events
 around every launch of further uncaptured steps, against 8 TB/s; its `traffic` is the
 HBM bytes per launch from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE
@@ -97,7 +98,7 @@ def adjoint_leg(steps: int, precision: int) -> dict:
     cost = backward wall time (recompute included) / plain forward wall time
     (pg_run with its captured step) over the same steps, both in the steady
     state of a loop that calls them repeatedly: the forward on a handle whose
-    step graphs a warm-up run captured, the backward on its second call (the
+    step graphs a warm-up run of as many steps captured, the backward on its second call (the
     first also captures the segment graphs; its time is reported apart).
     The tape_* keys: the same with every step's intermediates kept in HBM
     (ckpt_every 0, no recompute)."""
@@ -108,7 +109,7 @@ def adjoint_leg(steps: int, precision: int) -> dict:
     p = config_c5(precision=precision)
     target = gap_profile(p)
     d = Disk(p)
-    d.run(3, use_graph=True)                     # warm up kernels and capture the step's graphs
+    d.run(steps, use_graph=True)                 # warm up kernels and capture the graphs these steps need
     t0 = time.perf_counter()
     d.run(steps, use_graph=True)
     t_fwd = time.perf_counter() - t0
@@ -281,7 +282,7 @@ def fp64_leg(nr: int, nphi: int, steps: int) -> dict:
     p = config_c2(precision=8, xres=nr, yres=nphi)
     cells = nr * nphi
     d = Disk(p)
-    d.run(3, use_graph=True)
+    d.run(steps, use_graph=True)   # warm up, and capture the graphs these steps need
     t0 = time.perf_counter()
     d.run(steps, use_graph=True)
     el = time.perf_counter() - t0
@@ -349,7 +350,7 @@ def batched_leg(ndisk: int, steps: int, precision: int) -> dict:
     cells = sum(int(p.xres) * int(p.yres) for p in ps)
     b = Batch(ps)
     tune_ms = b.autotune(steps=3)
-    b.run(5)
+    b.run(steps)   # warm up, and capture the graphs these steps need; the looped disks likewise
     t0 = time.perf_counter()
     b.run(steps)
     tb = time.perf_counter() - t0
@@ -367,7 +368,7 @@ def batched_leg(ndisk: int, steps: int, precision: int) -> dict:
     tl = 0.0
     for p in ps:
         d = Disk(p)
-        d.run(5, use_graph=True)
+        d.run(steps, use_graph=True)
         t0 = time.perf_counter()
         d.run(steps, use_graph=True)
         tl += time.perf_counter() - t0
@@ -403,8 +404,11 @@ def main():
     graph = not a.no_graph
     d.run(a.warmup, use_graph=graph)
 
-    # timed region: K steps of the device loop (dt on the device), replaying
-    # the captured step; nothing else runs on the stream
+    # timed region: one run of K steps of the device loop (dt on the device),
+    # replaying captured steps.  The run holds what every run does once (the
+    # first step's CFL pass and viscosity, the copies of the control block and
+    # the step sizes) and the capture of a graph the warm-up did not need, so
+    # few steps show a longer step than many; nothing else runs on the stream
     t0 = time.perf_counter()
     dts = d.run(a.steps, use_graph=graph)
     t1 = time.perf_counter()
