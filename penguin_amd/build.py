@@ -72,16 +72,17 @@ ADJCHECK = os.path.join(HERE, "libpg_adjcheck.so")
 
 
 def build_adjcheck(verbose: bool = False, out: str = ADJCHECK) -> str:
-    """Host-only library evaluating the per-cell functions and their
-    adjoints in FP64 (pg_adjcheck.cpp), for the derivative checks of the
-    CPU test suite."""
-    cmd = [hipcc()] + flags() + ["-shared", "-x", "hip", os.path.join(CSRC, "pg_adjcheck.cpp"), "-o", out + ".tmp"]
+    """Host-only library for the CPU test suite: the per-cell functions and
+    their adjoints in FP64 (pg_adjcheck.cpp), and host code of the library over
+    a stand-in for the HIP calls it makes (pg_hostcheck.cpp)."""
+    srcs = [os.path.join(CSRC, f) for f in ("pg_adjcheck.cpp", "pg_hostcheck.cpp")]
+    cmd = [hipcc()] + flags() + ["-shared", "-x", "hip"] + srcs + ["-o", out + ".tmp"]
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         sys.stderr.write(r.stdout + r.stderr)
-        raise RuntimeError("hipcc failed on pg_adjcheck.cpp")
+        raise RuntimeError("hipcc failed on pg_adjcheck.cpp or pg_hostcheck.cpp")
     os.replace(out + ".tmp", out)
     return out
 

@@ -15,28 +15,34 @@
 #include <algorithm>
 #include <condition_variable>
 #include <cstddef>
+#include <cstdlib>
 #include <mutex>
 #include <thread>
 #include <vector>
 
 namespace pg {
 
-// The pinned pieces of one handle: at most NBUF x MOST bytes, allocated by the
-// first frame and freed with the handle.  One frame at a time (a handle
-// is used by one host thread).
+// The pieces of one handle: at most NBUF x MOST bytes, pinned (pageable where
+// the system gives no pinned memory), allocated by the first frame and freed
+// with the handle.  One frame at a time (a handle is used by one host thread).
 struct FrameBuf {
     static constexpr int NBUF = 3;
     static constexpr size_t LEAST = (size_t)1 << 20, MOST = (size_t)8 << 20;   // of a piece
     char* mem = nullptr;
+    bool pinned = false;
     size_t piece = 0;   // bytes of one piece
     int nbuf = 0;       // pieces held
     hipEvent_t ev[NBUF] = {nullptr, nullptr, nullptr};
 
-    void release() {
-        if (mem) (void)hipHostFree(mem);
+    void drop() {
+        if (mem && pinned) (void)hipHostFree(mem);
+        else std::free(mem);
         mem = nullptr;
         piece = 0;
         nbuf = 0;
+    }
+    void release() {
+        drop();
         for (hipEvent_t& e : ev) {
             if (e) (void)hipEventDestroy(e);
             e = nullptr;
@@ -55,14 +61,12 @@ struct FrameBuf {
         if (piece >= bytes && nbuf >= n) return hipSuccess;
         bytes = std::max(bytes, piece);   // disks of a batch share the buffers
         n = std::max(n, nbuf);
-        if (mem) (void)hipHostFree(mem);
-        mem = nullptr;
-        piece = 0;
-        nbuf = 0;
-        const hipError_t r = hipHostMalloc((void**)&mem, n * bytes, hipHostMallocDefault);
-        if (r != hipSuccess) {
-            mem = nullptr;
-            return r;
+        drop();
+        pinned = hipHostMalloc((void**)&mem, n * bytes, hipHostMallocDefault) == hipSuccess;
+        if (!pinned) {   // a frame can be read without: the copies are then staged by the runtime
+            (void)hipGetLastError();
+            mem = (char*)std::malloc(n * bytes);
+            if (!mem) return hipErrorOutOfMemory;
         }
         piece = bytes;
         nbuf = n;

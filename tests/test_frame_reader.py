@@ -1,0 +1,59 @@
+"""The frame reader (pg_frame.h) on the CPU, over a stand-in for the HIP calls
+it makes whose copies land at the earliest or at the latest moment a stream may
+choose: every cell arrives once whatever the shape, a second and third read
+through the same buffers too, and a read that fails ends, reports and leaves
+nothing behind."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from penguin_amd.build import ADJCHECK
+
+OUT_OF_MEMORY, INVALID_VALUE = 2, 1      # hipError_t
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return ctypes.CDLL(ADJCHECK)
+
+
+def _read(lib, rows, nx, nf, reads=1, late=0, refuse=0, fail=-1):
+    src = np.random.default_rng(rows + nx).standard_normal((nf, rows, nx)).astype(np.float32)
+    dst = np.zeros((nf, rows, nx))
+    stats = (ctypes.c_long * 6)()
+    err = lib.hostcheck_frame(ctypes.c_long(rows), ctypes.c_long(nx), nf, reads, late, refuse, fail,
+                              src.ctypes.data_as(ctypes.c_void_p), dst.ctypes.data_as(ctypes.c_void_p), stats)
+    return err, src, dst, dict(zip(("copies", "allocs", "most", "pinned", "events", "threads"), stats))
+
+
+# one piece by one thread, several pieces by one, several pieces by several
+# threads with a ragged last piece, rows longer than a piece
+SHAPES = [(7, 5, 3), (300, 260, 3), (301, 4001, 3), (3001, 701, 5), (3, 700001, 5)]
+
+
+@pytest.mark.parametrize("rows, nx, nf", SHAPES)
+@pytest.mark.parametrize("late", [0, 1])
+def test_every_cell_once(lib, rows, nx, nf, late):
+    err, src, dst, st = _read(lib, rows, nx, nf, reads=3, late=late)
+    assert err == 0
+    assert np.array_equal(dst, 3 * src.astype(np.float64))
+    assert st["pinned"] == 0 and st["events"] == 0, st
+
+
+@pytest.mark.parametrize("rows, nx, nf", SHAPES)
+@pytest.mark.parametrize("late", [0, 1])
+def test_without_pinned_memory(lib, rows, nx, nf, late):
+    err, src, dst, st = _read(lib, rows, nx, nf, reads=2, late=late, refuse=1)
+    assert err == 0 and st["allocs"] == 0
+    assert np.array_equal(dst, 2 * src.astype(np.float64))
+
+
+@pytest.mark.parametrize("rows, nx, nf", SHAPES)
+@pytest.mark.parametrize("late", [0, 1])
+def test_a_copy_that_fails(lib, rows, nx, nf, late):
+    copies = _read(lib, rows, nx, nf)[3]["copies"]
+    for fail in sorted({0, copies // 2, copies - 1}):
+        err, _, _, st = _read(lib, rows, nx, nf, reads=2, late=late, fail=fail)
+        assert err == INVALID_VALUE, fail
+        assert st["pinned"] == 0 and st["events"] == 0, st
