@@ -22,9 +22,10 @@
 
 namespace pg {
 
-// The pieces of one handle: at most NBUF x MOST bytes, pinned (pageable where
-// the system gives no pinned memory), allocated by the first frame and freed
-// with the handle.  One frame at a time (a handle is used by one host thread).
+// The pieces of one handle: at most NBUF x MOST bytes, pinned if there are
+// several (pageable where the system gives no pinned memory), allocated by the
+// first frame and freed with the handle.  One frame at a time (a handle is
+// used by one host thread).
 struct FrameBuf {
     static constexpr int NBUF = 3;
     static constexpr size_t LEAST = (size_t)1 << 20, MOST = (size_t)8 << 20;   // of a piece
@@ -48,7 +49,10 @@ struct FrameBuf {
             e = nullptr;
         }
     }
-    // n buffers of `bytes`; a frame of one piece needs neither more nor an event
+    // n buffers of `bytes`; a frame of one piece needs neither more nor an
+    // event, nor pinned memory, whose allocation and release cost as much as
+    // several such frames (64x128 FP32: first read 30 us, 53 pinned, every
+    // other 22 either way; 192x384, 0.9 MB: 111 and 127, then 104 and 84)
     hipError_t reserve(size_t bytes, int n) {
         for (hipEvent_t& e : ev)
             if (!e && n > 1) {
@@ -62,9 +66,9 @@ struct FrameBuf {
         bytes = std::max(bytes, piece);   // disks of a batch share the buffers
         n = std::max(n, nbuf);
         drop();
-        pinned = hipHostMalloc((void**)&mem, n * bytes, hipHostMallocDefault) == hipSuccess;
+        pinned = n > 1 && hipHostMalloc((void**)&mem, n * bytes, hipHostMallocDefault) == hipSuccess;
         if (!pinned) {   // a frame can be read without: the copies are then staged by the runtime
-            (void)hipGetLastError();
+            if (n > 1) (void)hipGetLastError();
             mem = (char*)std::malloc(n * bytes);
             if (!mem) return hipErrorOutOfMemory;
         }
@@ -97,9 +101,10 @@ hipError_t read_frame(FrameBuf& fb, hipStream_t s, const void* dev, size_t fstri
     auto buf = [&](size_t c) { return fb.mem + (c % FrameBuf::NBUF) * fb.piece; };
     auto fetch = [&](size_t c) {
         const size_t w = count(c) * row;
-        for (int f = 0; f < nf; ++f) {
-            const hipError_t e = hipMemcpyAsync(buf(c) + f * w, (const char*)dev + f * fstride + first(c) * row, w,
-                                                hipMemcpyDeviceToHost, s);
+        const bool whole = w == fstride;   // one piece of all fields: they adjoin on the device too
+        for (int f = 0; f < (whole ? 1 : nf); ++f) {
+            const hipError_t e = hipMemcpyAsync(buf(c) + f * w, (const char*)dev + f * fstride + first(c) * row,
+                                                whole ? nf * w : w, hipMemcpyDeviceToHost, s);
             if (e != hipSuccess) return e;
         }
         return npiece > 1 ? hipEventRecord(fb.ev[c % FrameBuf::NBUF], s) : hipSuccess;

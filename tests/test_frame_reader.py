@@ -57,3 +57,10 @@ def test_a_copy_that_fails(lib, rows, nx, nf, late):
         err, _, _, st = _read(lib, rows, nx, nf, reads=2, late=late, fail=fail)
         assert err == INVALID_VALUE, fail
         assert st["pinned"] == 0 and st["events"] == 0, st
+
+
+@pytest.mark.parametrize("rows, nx, nf", [(7, 5, 3), (128, 64, 3), (330, 260, 3)])
+def test_a_small_frame_is_one_copy_without_pinned_memory(lib, rows, nx, nf):
+    err, src, dst, st = _read(lib, rows, nx, nf, reads=2)
+    assert err == 0 and np.array_equal(dst, 2 * src.astype(np.float64))
+    assert st["copies"] == 1 and st["allocs"] == 0 and st["threads"] == 1, st
