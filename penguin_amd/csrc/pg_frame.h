@@ -22,15 +22,17 @@
 
 namespace pg {
 
-// The pieces of one handle: at most NBUF x MOST bytes, pinned if there are
-// several (pageable where the system gives no pinned memory), allocated by the
-// first frame and freed with the handle.  One frame at a time (a handle is
-// used by one host thread).
+// The pieces of one handle: at most NBUF x MOST bytes, allocated by the first
+// frame, pinned if it reads enough through them and the system gives pinned
+// memory, and freed with the handle.  One frame at a time (a handle is used by
+// one host thread).
 struct FrameBuf {
     static constexpr int NBUF = 3;
     static constexpr size_t LEAST = (size_t)1 << 20, MOST = (size_t)8 << 20;   // of a piece
+    static constexpr size_t PIN_FROM = (size_t)16 << 20;   // bytes read
     char* mem = nullptr;
-    bool pinned = false;
+    bool pinned = false, refused = false;
+    size_t read = 0;    // bytes of all frames so far
     size_t piece = 0;   // bytes of one piece
     int nbuf = 0;       // pieces held
     hipEvent_t ev[NBUF] = {nullptr, nullptr, nullptr};
@@ -49,11 +51,16 @@ struct FrameBuf {
             e = nullptr;
         }
     }
-    // n buffers of `bytes`; a frame of one piece needs neither more nor an
-    // event, nor pinned memory, whose allocation and release cost as much as
-    // several such frames (64x128 FP32: first read 30 us, 53 pinned, every
-    // other 22 either way; 192x384, 0.9 MB: 111 and 127, then 104 and 84)
-    hipError_t reserve(size_t bytes, int n) {
+    // n buffers of `bytes` for a frame of `frame` bytes; a frame of one piece
+    // needs neither more nor an event, nor pinned memory, whose allocation and
+    // release cost as much as several such frames (64x128 FP32: first read 30
+    // us, 53 pinned, every other 22 either way; 192x384, 0.9 MB: 111 and 127,
+    // then 104 and 84).  Pieces are pinned once the handle has read 16 MB, this
+    // frame included: three of 1 MB take 0.1-1 ms to allocate and gain 0.05 ms
+    // for each MB read (256x512 FP32, 1.6 MB: first read 250 us, 200-1200
+    // pinned, then 230 and 165 a frame; 1024x3072, 38 MB: 4.7 ms, pinned 3.6,
+    // then 2.9).
+    hipError_t reserve(size_t bytes, int n, size_t frame) {
         for (hipEvent_t& e : ev)
             if (!e && n > 1) {
                 const hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
@@ -62,13 +69,16 @@ struct FrameBuf {
                     return r;
                 }
             }
-        if (piece >= bytes && nbuf >= n) return hipSuccess;
+        read += frame;
+        const bool pin = pinned || (n > 1 && read >= PIN_FROM && !refused);
+        if (piece >= bytes && nbuf >= n && pin == pinned) return hipSuccess;
         bytes = std::max(bytes, piece);   // disks of a batch share the buffers
         n = std::max(n, nbuf);
         drop();
-        pinned = n > 1 && hipHostMalloc((void**)&mem, n * bytes, hipHostMallocDefault) == hipSuccess;
+        pinned = pin && hipHostMalloc((void**)&mem, n * bytes, hipHostMallocDefault) == hipSuccess;
         if (!pinned) {   // a frame can be read without: the copies are then staged by the runtime
-            if (n > 1) (void)hipGetLastError();
+            if (pin) (void)hipGetLastError();
+            refused = pin;
             mem = (char*)std::malloc(n * bytes);
             if (!mem) return hipErrorOutOfMemory;
         }
@@ -94,7 +104,7 @@ hipError_t read_frame(FrameBuf& fb, hipStream_t s, const void* dev, size_t fstri
     const size_t bytes = std::min(FrameBuf::MOST, std::max(FrameBuf::LEAST, rows * row * nf / 16));
     const size_t per = std::min(rows, std::max<size_t>(1, bytes / (row * nf)));   // rows of a piece
     const size_t npiece = (rows + per - 1) / per;
-    hipError_t err = fb.reserve(per * row * nf, npiece > 1 ? FrameBuf::NBUF : 1);
+    hipError_t err = fb.reserve(per * row * nf, npiece > 1 ? FrameBuf::NBUF : 1, rows * row * nf);
     if (err != hipSuccess) return err;
     auto first = [&](size_t c) { return c * per; };
     auto count = [&](size_t c) { return std::min(rows, (c + 1) * per) - c * per; };
