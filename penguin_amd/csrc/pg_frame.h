@@ -22,8 +22,8 @@
 
 namespace pg {
 
-// The pieces of one handle: at most NBUF x MOST bytes, allocated by the first
-// frame, pinned if it reads enough through them and the system gives pinned
+// The pieces of one handle: at most NBUF of MOST bytes, or of one row of all
+// fields where that is more, allocated by the first frame, pinned if it reads enough through them and the system gives pinned
 // memory, and freed with the handle.  One frame at a time (a handle is used by
 // one host thread).
 struct FrameBuf {
@@ -35,6 +35,7 @@ struct FrameBuf {
     size_t read = 0;    // bytes of all frames so far
     size_t piece = 0;   // bytes of one piece
     int nbuf = 0;       // pieces held
+    size_t threads = 0; // that converted the last frame
     hipEvent_t ev[NBUF] = {nullptr, nullptr, nullptr};
 
     void drop() {
@@ -124,7 +125,8 @@ hipError_t read_frame(FrameBuf& fb, hipStream_t s, const void* dev, size_t fstri
     // is still spinning: a pass that reads 24 disks of 33k-786k cells and has
     // torch convert each takes 142 ms, with threads of 128k cells 164, of 32k 206.
     const size_t hw = std::max(1u, std::thread::hardware_concurrency());
-    const size_t want = std::min<size_t>(std::min<size_t>(hw, 8), std::max<size_t>(1, rows * nx / 262144));
+    // A thread takes whole rows of a piece, so no more threads than those.
+    const size_t want = std::min({hw, (size_t)8, per, std::max<size_t>(1, rows * nx / 262144)});
     std::mutex mu;
     std::condition_variable cv;
     size_t ready = 0;                      // pieces that have arrived
@@ -157,7 +159,7 @@ hipError_t read_frame(FrameBuf& fb, hipStream_t s, const void* dev, size_t fstri
         } catch (...) {
         }
     }
-    nt = std::max<size_t>(1, th.size());
+    fb.threads = nt = std::max<size_t>(1, th.size());
     size_t asked = 0;
     for (size_t c = 0; c < npiece && err == hipSuccess; ++c) {
         // keep the free buffers on their way; piece `asked` takes the buffer of

@@ -100,7 +100,8 @@ extern "C" {
 // converted to doubles at dst; the last one fails at its fail_copy-th copy if
 // that is not negative.  Returns the last read's error.  stats: copies of the
 // last read, pinned allocations, most pinned bytes at once, pinned bytes and
-// events left after the release, threads that converted in the last read.
+// events left after the release, threads that converted rows in the last read
+// and threads that it was given.
 int hostcheck_frame(long rows, long nx, int nf, int reads, int late, int refuse_pinned, int fail_copy,
                     const float* src, double* dst, long* stats) {
     fake::dev = fake::Device();
@@ -133,6 +134,7 @@ int hostcheck_frame(long rows, long nx, int nf, int reads, int late, int refuse_
     stats[3] = fake::dev.pinned;
     stats[4] = fake::dev.nevent;
     stats[5] = (long)ids.size();
+    stats[6] = (long)fb.threads;
     return (int)e;
 }
 

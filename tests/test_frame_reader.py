@@ -21,10 +21,11 @@ def lib():
 def _read(lib, rows, nx, nf, reads=1, late=0, refuse=0, fail=-1):
     src = np.random.default_rng(rows + nx).standard_normal((nf, rows, nx)).astype(np.float32)
     dst = np.zeros((nf, rows, nx))
-    stats = (ctypes.c_long * 6)()
+    stats = (ctypes.c_long * 7)()
     err = lib.hostcheck_frame(ctypes.c_long(rows), ctypes.c_long(nx), nf, reads, late, refuse, fail,
                               src.ctypes.data_as(ctypes.c_void_p), dst.ctypes.data_as(ctypes.c_void_p), stats)
-    return err, src, dst, dict(zip(("copies", "allocs", "most", "pinned", "events", "threads"), stats))
+    return err, src, dst, dict(zip(("copies", "allocs", "most", "pinned", "events", "threads", "given"),
+                                     stats))
 
 
 # one piece by one thread, several pieces by one, several pieces by several
@@ -74,3 +75,14 @@ def test_pieces_are_pinned_once_16_mb_are_read(lib, rows, nx, nf, pins_at):
             err, src, dst, st = _read(lib, rows, nx, nf, reads=reads, late=1)
             assert err == 0 and np.array_equal(dst, reads * src.astype(np.float64))
             assert st["allocs"] == (reads >= pins_at) and st["pinned"] == 0, st
+
+
+# rows of 14, 0.6 and 0.014 MB: a piece holds 1, 4 and 187 of them
+@pytest.mark.parametrize("rows, nx, nf, per", [(6, 700001, 5, 1), (74, 30001, 5, 4), (3001, 701, 5, 187)])
+def test_threads_and_pieces_follow_the_rows(lib, rows, nx, nf, per):
+    err, src, dst, st = _read(lib, rows, nx, nf, reads=2, late=1)
+    assert err == 0 and np.array_equal(dst, 2 * src.astype(np.float64))
+    assert 1 <= st["threads"] <= st["given"] <= min(8, per), st
+    row = 4 * nx * nf
+    assert st["copies"] == nf * -(-rows // per), st
+    assert st["most"] == 3 * per * row and per * row <= max(8 << 20, row), st
