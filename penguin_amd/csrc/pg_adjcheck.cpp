@@ -90,4 +90,7 @@ void adjc_slopes_f32(const float* x, float* y) {
     slopes(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7], x[8], x[9], x[10], x[11], y[0], y[1]);
 }
 
+// pem_series in FP64
+double adjc_pem_series(double eta, double x) { return pem_series(eta, x); }
+
 }  // extern "C"

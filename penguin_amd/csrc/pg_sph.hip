@@ -205,16 +205,7 @@ __device__ __forceinline__ void edge_means(real x, const Par<real> (&P)[N], real
         const real E = FM<real>::exp(eta * (z ? lx : ly));
         const real ex = eta * x;
         real v = z ? E : FM<real>::div(y * (E - real(1)), ex) + real(1);
-        if (P[f].pl && !z && !(ex > real(0.001))) {
-            real t = (eta + real(1)) * x * real(0.5);
-            v = t;
-            t *= -(eta - real(1)) * x * real(1.0 / 3.0);
-            v += t;
-            t *= -(eta - real(2)) * x * real(0.25);
-            v += t;
-            t *= -(eta - real(3)) * x * real(0.2);
-            v += t;
-        }
+        if (P[f].pl && !z && !(ex > real(0.001))) v = pem_series(eta, x);
         m[f] = P[f].pl ? (P[f].a - S) + S * v : m[f];
     }
 }
