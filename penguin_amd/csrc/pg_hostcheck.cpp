@@ -1,5 +1,6 @@
 // pg_hostcheck.cpp -- host code of the library run on the CPU, for its tests:
-// the frame reader (pg_frame.h) over a stand-in for the HIP calls it makes.
+// the frame reader (pg_frame.h) over a stand-in for the HIP calls it makes, and
+// the choice of the 3D radial sweep's tile.
 // Part of libpg_adjcheck.so; the product library does not contain it.
 #include <hip/hip_runtime.h>
 
@@ -93,6 +94,7 @@ hipError_t last_error() { return hipSuccess; }
 #define hipStreamSynchronize fake::stream_wait
 #define hipGetLastError fake::last_error
 #include "pg_frame.h"
+#include "pg_sph.h"
 
 extern "C" {
 
@@ -136,6 +138,15 @@ int hostcheck_frame(long rows, long nx, int nf, int reads, int late, int refuse_
     stats[5] = (long)ids.size();
     stats[6] = (long)fb.threads;
     return (int)e;
+}
+
+// Cells of a segment, rows of a block and row multiplier of the radial sweep of
+// a disk of nx radii in `rows` rows, es bytes a real.
+void hostcheck_radial_tile(int nx, long rows, int es, int* out) {
+    const pg::RadialTile t = pg::radial_tile(nx, rows, es);
+    out[0] = t.tx;
+    out[1] = t.xr;
+    out[2] = t.xm;
 }
 
 }  // extern "C"

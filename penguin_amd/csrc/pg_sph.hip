@@ -51,7 +51,6 @@ namespace {
 
 constexpr int NF = 5;            // rho, p, u, vp, w
 constexpr int SPH_BT = 256;      // threads per block of the pointwise kernels
-constexpr int SPH_BT2 = 512;     // threads per block of the sweeps (about one element each)
 constexpr int SPH_R = 8;         // rows per strided-sweep block
 // azimuthal segment per block: with its 6 halo rows, 8 radii x 64 slots fill
 // a 512-thread block (and two passes of a 256-thread one) exactly (64 rows:
@@ -100,43 +99,8 @@ struct SphK {
     real dy, idy;
     double dy_d;
     real gam;
-    int tx, xr;   // radial sweep: cells of a segment, rows of a block (radial_tile)
-    int xm;       // (1 << 20) / (tx + 2 NPAD) + 1: t / (tx + 2 NPAD) = (t * xm) >> 20 for t < SPH_BT2
+    int tx, xr, xm;   // tile of the radial sweep (RadialTile)
 };
-
-// Tile of the radial sweep: xr rows x a segment of tx cells.  The row is cut
-// into equal segments, and as many rows as fit SPH_BT2 threads (one per slot,
-// segment + 2 NPAD slots a row; half as many in FP64, whose PEM4 sweep needs
-// 160 VGPRs: 84 us against 127 on a 96x192x32 disk) make a block; of all cuts
-// the one that puts the most cells into a block's threads, so that few lanes issue instructions
-// for halo cells or for nothing (a 384-radius row: five rows of four 102-slot
-// segments fill 480 of 512 lanes with cells, one row's two 198-slot segments
-// 192 of 256: radial sweep of the 384x1536x64 disk 1210 -> 1140 us, its lanes
-// in use 75 -> 88 %).  A small disk takes fewer rows, down to one, so that the
-// blocks still cover the chip's 256 CUs eight times (a 101x190x33 disk is 1 %
-// slower with four rows in 1568 blocks than with three in 2090).
-struct RadialTile {
-    int tx, xr;
-};
-inline RadialTile radial_tile(int nx, long rows, int es) {
-    const int most_threads = es == 8 ? SPH_BT2 / 2 : SPH_BT2;
-    RadialTile best{0, 0};
-    double most = 0.0;
-    for (int parts = (nx + most_threads - 2 * NPAD - 1) / (most_threads - 2 * NPAD); parts <= nx; ++parts) {
-        const int tx = (nx + parts - 1) / parts;
-        if (best.tx && tx < 32) break;   // the halo alone is 16 % there
-        const long nseg = (nx + tx - 1) / tx;
-        int xr = most_threads / (tx + 2 * NPAD);
-        while (xr > 1 && nseg * ((rows + xr - 1) / xr) < 2048) --xr;
-        const int threads = (xr * (tx + 2 * NPAD) + 63) / 64 * 64;
-        const double use = (double)nx * xr / ((double)nseg * threads);
-        if (use > most) {
-            most = use;
-            best = RadialTile{tx, xr};
-        }
-    }
-    return best;
-}
 
 template <typename real>
 struct PlanetS {   // planet for the spherical force: mass, radius, angle, softening
@@ -1126,7 +1090,8 @@ struct Sph {
     void* rate = nullptr;
     void* rate_h = nullptr;     // pinned: the reduced rate
     int rate_n = 0;             // blocks' maxima in rate
-    FrameBuf frame;             // pinned pieces of a state being read back
+    FrameBuf frame;             // pieces of a state being read back
+    RadialTile rt{};            // of the radial sweep
     size_t tab_off[16] = {0};
     std::vector<double> xa, xv, ya, yv, za, zv, vbg, rot, rcyl;
     std::vector<double> xgh;    // radial ghost states (rho, p, u, v, w) [field][ghost 0..5][polar k], FP64
@@ -1168,10 +1133,9 @@ SphK<real> kargs(Sph* s, int in, int out) {
     a.idy = (real)(1.0 / dy);
     a.dy_d = dy;
     a.gam = (real)s->P.gam;
-    const RadialTile rt = radial_tile(s->nx, (long)s->ny * s->nz, (int)sizeof(real));
-    a.tx = rt.tx;
-    a.xr = rt.xr;
-    a.xm = (1 << 20) / (rt.tx + 2 * NPAD) + 1;
+    a.tx = s->rt.tx;
+    a.xr = s->rt.xr;
+    a.xm = s->rt.xm;
     return a;
 }
 
@@ -1609,6 +1573,7 @@ int sph_create(const pg_params& P, Sph** out) {
     s->nx = P.xres; s->ny = P.yres; s->nz = P.zres;
     s->N = (size_t)P.xres * P.yres * P.zres;
     s->es = P.precision;
+    s->rt = radial_tile(s->nx, (long)s->ny * s->nz, s->es);
     rc = P.precision == 8 ? create_t<double>(s) : create_t<float>(s);
     if (rc) {
         sph_destroy(s);
