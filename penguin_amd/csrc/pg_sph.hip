@@ -109,13 +109,17 @@ struct PlanetS {   // planet for the spherical force: mass, radius, angle, softe
 
 // ----------------------------------------------------- reconstruction
 // The natural logarithm of a fraction in [0, 1] (__logf of a float argument,
-// PEM.cu:13,29) and the exponential of a multiple of it.  FP32: the hardware
-// base-2 logarithm times ln 2 in two parts, as __logf forms it, without its
-// scaling of denormal arguments (their powers here, above the second, are zero
-// either way) and with a finite number for the logarithm of zero, which every
-// power also takes to zero.  FP64 takes the float logarithm correctly rounded
-// (the double logarithm of the float argument, rounded to float), as the
-// oracle does.
+// PEM.cu:13,29).  FP32: the hardware's base-2 logarithm times ln 2 held in two
+// parts, with the first product's remainder by a fused multiply-add (the exact
+// product of Dekker, Numer. Math. 18, 1971).  The remainder enters the sum twice,
+// by itself and through the outer product, which does not round: at most 0.95
+// ulp, where h plus the inner sum would give 0.50.  It stays so because 3D FP32
+// states hang on the last bit (near the planet a change of it grows to 1e-3 in
+// 120 steps) and all of them were computed with it.  Denormal arguments are not
+// scaled (their powers here, above the second, are zero either way), and the
+// logarithm of zero is a finite number, which every power also takes to zero.
+// FP64 takes the float logarithm correctly rounded (the double logarithm of the
+// float argument, rounded to float), as the oracle does.
 template <typename real> __device__ __forceinline__ real flog(real x);
 template <> __device__ __forceinline__ float flog<float>(float x) {
     const float r = fmaxf(__builtin_amdgcn_logf(x), -1024.0f), ln2 = 0x1.62e42ep-1f, ln2_lo = 0x1.efa39ep-25f;
