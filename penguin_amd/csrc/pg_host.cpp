@@ -333,7 +333,7 @@ struct Group {
     // pinned host staging for results read back after a run (the step sizes)
     double* stage = nullptr;
     size_t stage_bytes = 0;
-    FrameBuf frame;              // pinned pieces of a state being read back
+    FrameBuf frame;              // pieces of a state being read back
 
     int par() const { return gpar | (dpar << 1); }
     int ndisk() const { return (int)disks.size(); }
@@ -367,9 +367,12 @@ struct Group {
 };
 
 // Steps of a captured graph, longest first.  The first node of a graph waits
-// about 5 us for the launch, the others 1-2 us for the node before: a step of
-// its own 64x128 disk takes 26.2 us in graphs of one step, 21.4 in graphs of 8,
-// 24 disks 326 us and 314.
+// about 5 us for the launch, the others 1-2 us for the node before: a step of a
+// 64x128 disk takes 26.2 us in graphs of one step, 21.4 in these, of 24 disks
+// 326 and 315.  A captured step costs about 20 us once, which a new handle's
+// first run earns back: of 5, 20 and 100 steps of the 64x128 disk it takes 0.33,
+// 0.76 and 2.5 ms, every later one 0.17, 0.48 and 2.2 (in graphs of one step,
+// with the kernels of that time, 0.34, 0.83 and 3.4, then 0.21, 0.70 and 3.3).
 constexpr int GRAPH_STEPS[] = {16, 4, 1};
 
 struct AdjWork;
