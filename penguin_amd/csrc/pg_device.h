@@ -69,17 +69,26 @@ template <> struct FM<double> {
 };
 
 // ---------------------------------------------------------------- helpers
-// A minimum of two and a zero that together keep a value which is not a number:
-// in FP32 by the minimum itself, one instruction like the one that drops it
-// (v_minimum3_f32); FP64 has none, so there the zero is x - x.
-template <typename real> struct MinNan;
-template <> struct MinNan<float> {
+// What keeps a value that is not a number in the limiter below: in FP32 a minimum
+// that does, one instruction like the one that drops it (v_minimum3_f32); FP64
+// has none, so there the limiter's factor, (d > 0 ? 1 - flat : 0) elsewhere, takes
+// x - x for the zero, and without flattening only in its upper word.
+template <typename real> struct KeepNan;
+template <> struct KeepNan<float> {
     static PG_HD float min(float a, float b) { return __builtin_elementwise_minimum(a, b); }
-    static PG_HD float zero(float) { return 0.0f; }
+    static PG_HD float factor(float d, float flat) { return d > 0.0f ? 1.0f - flat : 0.0f; }
 };
-template <> struct MinNan<double> {
+template <> struct KeepNan<double> {
     static PG_HD double min(double a, double b) { return fmin(a, b); }
-    static PG_HD double zero(double x) { return x - x; }
+    static PG_HD double factor(double d, double flat) {
+#ifdef __HIP_DEVICE_COMPILE__
+        if (__builtin_constant_p(flat) && flat == 0.0) {
+            const int hi = d > 0.0 ? __double2hiint(1.0) : __double2hiint(d - d);
+            return __hiloint2double(hi, 0);   // a quiet NaN's upper word is one by itself
+        }
+#endif
+        return d > 0.0 ? 1.0 - flat : d - d;
+    }
 };
 // A product that is rounded before it is added to anything, where the compiler
 // could otherwise contract it into a fused multiply-add in one kernel and not in
@@ -147,10 +156,10 @@ PG_HD void slopes_d(real d0, real d1, real d2, real d3,
     real l = fmin(fabs(wl0 * d0 + wl1 * d1 + wl2 * d2), fabs(d1));
     real r = fmin(fabs(wr0 * d1 + wr1 * d2 + wr2 * d3), fabs(d2));
     const real d12 = d1 * d2;
-    const real fk = copysign(d12 > real(0) ? real(1) - flat : MinNan<real>::zero(d12), d1);
+    const real fk = copysign(KeepNan<real>::factor(d12, flat), d1);
     const real l2 = l + l, r2 = r + r;
-    l = fk * MinNan<real>::min(l, r2);
-    r = fk * MinNan<real>::min(r, l2);
+    l = fk * KeepNan<real>::min(l, r2);
+    r = fk * KeepNan<real>::min(r, l2);
     sL = l;
     sR = r;
 }
