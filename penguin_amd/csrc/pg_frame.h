@@ -29,7 +29,7 @@ namespace pg {
 struct FrameBuf {
     static constexpr int NBUF = 3;
     static constexpr size_t LEAST = (size_t)1 << 20, MOST = (size_t)8 << 20;   // of a piece
-    static constexpr size_t PIN_FROM = (size_t)16 << 20;   // bytes read
+    static constexpr size_t PIN_FROM = (size_t)4 << 20;   // bytes read
     char* mem = nullptr;
     bool pinned = false, refused = false;
     size_t read = 0;    // bytes of all frames so far
@@ -56,11 +56,11 @@ struct FrameBuf {
     // needs neither more nor an event, nor pinned memory, whose allocation and
     // release cost as much as several such frames (64x128 FP32: first read 30
     // us, 53 pinned, every other 22 either way; 192x384, 0.9 MB: 111 and 127,
-    // then 104 and 84).  Pieces are pinned once the handle has read 16 MB, this
-    // frame included: three of 1 MB take 0.1-1 ms to allocate and gain 0.05 ms
-    // for each MB read (256x512 FP32, 1.6 MB: first read 250 us, 200-1200
-    // pinned, then 230 and 165 a frame; 1024x3072, 38 MB: 4.7 ms, pinned 3.6,
-    // then 2.9).
+    // then 104 and 84).  Pieces are pinned once the handle has read 4 MB, this
+    // frame included: three of 1 MB take 0.1-1 ms to allocate and gain 0.05-0.1
+    // ms for each MB read (256x512 FP32, 1.6 MB: first read 250 us, pinned
+    // 200-1200, then 230 and 165 a frame; 333x777 FP64 gas and dust, 12 MB: 1.9
+    // ms, pinned 1.3; 1024x3072 FP32 gas, 38 MB: 4.7 ms, pinned 3.6, then 2.9).
     hipError_t reserve(size_t bytes, int n, size_t frame) {
         for (hipEvent_t& e : ev)
             if (!e && n > 1) {

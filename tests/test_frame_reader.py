@@ -67,9 +67,9 @@ def test_a_small_frame_is_one_copy_without_pinned_memory(lib, rows, nx, nf):
     assert st["copies"] == 1 and st["allocs"] == 0 and st["threads"] == 1, st
 
 
-# 14 MB: the second read pins; 42 MB: the first does; 1.9 MB: the ninth
-@pytest.mark.parametrize("rows, nx, nf, pins_at", [(301, 4001, 3, 2), (3001, 701, 5, 1), (401, 401, 3, 9)])
-def test_pieces_are_pinned_once_16_mb_are_read(lib, rows, nx, nf, pins_at):
+# 42 and 7 MB: the first read; 2.4 MB: the second; 1.9 MB: the third
+@pytest.mark.parametrize("rows, nx, nf, pins_at", [(3001, 701, 5, 1), (301, 2001, 3, 1), (500, 401, 3, 2), (401, 401, 3, 3)])
+def test_pieces_are_pinned_once_4_mb_are_read(lib, rows, nx, nf, pins_at):
     for reads in (pins_at - 1, pins_at, pins_at + 2):
         if reads:
             err, src, dst, st = _read(lib, rows, nx, nf, reads=reads, late=1)

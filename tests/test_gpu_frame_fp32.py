@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 EPS = np.finfo(np.float32).eps
 
 
-# 0.2, 3, 9 (gas and dust: 16 MB at the second read) and 25 MB a fluid
+# 0.15 (never pinned), 3 (at the second read), 9 and 25 MB a fluid
 @pytest.mark.parametrize("nr, nphi", [(41, 301), (257, 1023), (600, 1300), (701, 3001)])
 @pytest.mark.parametrize("dust", [0, 1])
 def test_frame_2d_fp32(nr, nphi, dust):
