@@ -58,9 +58,8 @@ int pg_destroy(pg_handle* h);
 /* Copy the interior state to/from host FP64 buffers (main.cu:61-104).
    gas: 5*xres*yres*zres doubles (rho,p,u,v,w); dust: 4*xres*yres (rho,u,v,w)
    or NULL.  On set, p is ignored under EOS_flag 0 (it is c_s^2(R)*rho).
-   The first get keeps up to 24 MB of host memory with the handle for those
-   that follow (or three rows of all fields, if they are longer), pinned once
-   4 MB have been read and if there is any to be had. */
+   Gets keep up to 24 MB of host memory with the handle (or three rows of all
+   fields, if they are longer), pinned above 1 MB if there is any to be had. */
 int pg_get_state(pg_handle* h, double* gas, double* dust);
 int pg_set_state(pg_handle* h, const double* gas, const double* dust);
 

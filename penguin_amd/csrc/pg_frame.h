@@ -23,25 +23,25 @@
 namespace pg {
 
 // The pieces of one handle: at most NBUF of MOST bytes, or of one row of all
-// fields where that is more, allocated by the first frame, pinned if it reads enough through them and the system gives pinned
-// memory, and freed with the handle.  One frame at a time (a handle is used by
-// one host thread).
+// fields where that is more, allocated by the first frame that needs them and
+// freed with the handle.  One frame at a time (a handle is used by one host
+// thread).
 struct FrameBuf {
     static constexpr int NBUF = 3;
     static constexpr size_t LEAST = (size_t)1 << 20, MOST = (size_t)8 << 20;   // of a piece
-    static constexpr size_t PIN_FROM = (size_t)4 << 20;   // bytes read
-    char* mem = nullptr;
-    bool pinned = false, refused = false;
-    size_t read = 0;    // bytes of all frames so far
+    char* mem[NBUF] = {nullptr, nullptr, nullptr};
+    bool pinned = false;
     size_t piece = 0;   // bytes of one piece
     int nbuf = 0;       // pieces held
     size_t threads = 0; // that converted the last frame
     hipEvent_t ev[NBUF] = {nullptr, nullptr, nullptr};
 
     void drop() {
-        if (mem && pinned) (void)hipHostFree(mem);
-        else std::free(mem);
-        mem = nullptr;
+        for (char*& m : mem) {
+            if (m && pinned) (void)hipHostFree(m);
+            else std::free(m);
+            m = nullptr;
+        }
         piece = 0;
         nbuf = 0;
     }
@@ -52,40 +52,43 @@ struct FrameBuf {
             e = nullptr;
         }
     }
-    // n buffers of `bytes` for a frame of `frame` bytes; a frame of one piece
-    // needs neither more nor an event, nor pinned memory, whose allocation and
-    // release cost as much as several such frames (64x128 FP32: first read 30
-    // us, 53 pinned, every other 22 either way; 192x384, 0.9 MB: 111 and 127,
-    // then 104 and 84).  Pieces are pinned once the handle has read 4 MB, this
-    // frame included: three of 1 MB take 0.1-1 ms to allocate and gain 0.05-0.1
-    // ms for each MB read (256x512 FP32, 1.6 MB: first read 250 us, pinned
-    // 200-1200, then 230 and 165 a frame; 333x777 FP64 gas and dust, 12 MB: 1.9
-    // ms, pinned 1.3; 1024x3072 FP32 gas, 38 MB: 4.7 ms, pinned 3.6, then 2.9).
-    hipError_t reserve(size_t bytes, int n, size_t frame) {
-        for (hipEvent_t& e : ev)
-            if (!e && n > 1) {
-                const hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
-                if (r != hipSuccess) {
-                    e = nullptr;
-                    return r;
-                }
+    bool allocate(size_t bytes, int n, bool pin) {
+        pinned = pin;
+        for (int k = 0; k < n; ++k) {
+            if (pin ? hipHostMalloc((void**)&mem[k], bytes, hipHostMallocDefault) != hipSuccess
+                    : !(mem[k] = (char*)std::malloc(bytes))) {
+                mem[k] = nullptr;
+                if (pin) (void)hipGetLastError();
+                drop();
+                return false;
             }
-        read += frame;
-        const bool pin = pinned || (n > 1 && read >= PIN_FROM && !refused);
-        if (piece >= bytes && nbuf >= n && pin == pinned) return hipSuccess;
-        bytes = std::max(bytes, piece);   // disks of a batch share the buffers
-        n = std::max(n, nbuf);
-        drop();
-        pinned = pin && hipHostMalloc((void**)&mem, n * bytes, hipHostMallocDefault) == hipSuccess;
-        if (!pinned) {   // a frame can be read without: the copies are then staged by the runtime
-            if (pin) (void)hipGetLastError();
-            refused = pin;
-            mem = (char*)std::malloc(n * bytes);
-            if (!mem) return hipErrorOutOfMemory;
         }
         piece = bytes;
         nbuf = n;
-        return hipSuccess;
+        return true;
+    }
+    // n pieces of `bytes`; a frame of one piece needs neither more nor an event,
+    // nor pinned memory, whose allocation and release cost as much as several
+    // such frames (64x128 FP32: first read 30 us, 53 pinned, every other 22
+    // either way; 192x384, 0.9 MB: 111 and 127, then 104 and 84).  A piece is an
+    // allocation of its own: up to 1 MB they take some 35 us each, one of 3 MB
+    // takes 0.1 or 1 ms (first read of a 256x512 FP32 disk, 1.6 MB: 210-240 us,
+    // with its pieces in one block 200 or 820-1140; of a 256x512 FP64 one 290
+    // and 280 or 1410).  Without pinned memory the runtime stages the copies.
+    hipError_t reserve(size_t bytes, int n) {
+        for (int k = 0; k < n && n > 1; ++k)
+            if (!ev[k]) {
+                const hipError_t r = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+                if (r != hipSuccess) {
+                    ev[k] = nullptr;
+                    return r;
+                }
+            }
+        if (piece >= bytes && nbuf >= n) return hipSuccess;
+        bytes = std::max(bytes, piece);   // disks of a batch share the pieces
+        n = std::max(n, nbuf);
+        drop();
+        return (n > 1 && allocate(bytes, n, true)) || allocate(bytes, n, false) ? hipSuccess : hipErrorOutOfMemory;
     }
 };
 
@@ -101,15 +104,16 @@ hipError_t read_frame(FrameBuf& fb, hipStream_t s, const void* dev, size_t fstri
     // sixteen pieces or pieces of MOST: pinned pages cost the first frame about
     // 0.2 ms a megabyte, and small pieces more waits (the 1.5 GB frame: 29 ms
     // with 8 MB pieces, 45 with 2 MB; the first frame of a 512x1024 FP64 disk
-    // 2.5 ms slower with 4 MB pieces than with 1 MB)
+    // 2.5 ms slower with 4 MB pieces than with 1 MB; every frame of a 256x512
+    // FP32 disk 240 us with pieces of a third of a megabyte, 165 with 1 MB)
     const size_t bytes = std::min(FrameBuf::MOST, std::max(FrameBuf::LEAST, rows * row * nf / 16));
     const size_t per = std::min(rows, std::max<size_t>(1, bytes / (row * nf)));   // rows of a piece
     const size_t npiece = (rows + per - 1) / per;
-    hipError_t err = fb.reserve(per * row * nf, npiece > 1 ? FrameBuf::NBUF : 1, rows * row * nf);
+    hipError_t err = fb.reserve(per * row * nf, (int)std::min<size_t>(npiece, FrameBuf::NBUF));
     if (err != hipSuccess) return err;
     auto first = [&](size_t c) { return c * per; };
     auto count = [&](size_t c) { return std::min(rows, (c + 1) * per) - c * per; };
-    auto buf = [&](size_t c) { return fb.mem + (c % FrameBuf::NBUF) * fb.piece; };
+    auto buf = [&](size_t c) { return fb.mem[c % FrameBuf::NBUF]; };
     auto fetch = [&](size_t c) {
         const size_t w = count(c) * row;
         const bool whole = w == fstride;   // one piece of all fields: they adjoin on the device too

@@ -28,7 +28,7 @@ struct Device {
     size_t done = 0;                          // copies of the queue that have happened
     std::vector<size_t> mark = std::vector<size_t>(64, 0);   // per event: the queue's length at its record
     int nevent = 0, ncopy = 0, nalloc = 0;
-    long pinned = 0, most = 0;                // bytes allocated now, and ever at once
+    long pinned = 0, most = 0, block = 0;     // bytes allocated now, ever at once, and in one block
     std::vector<std::pair<void*, size_t>> live;
 } dev;
 
@@ -36,12 +36,13 @@ void run_to(size_t n) {
     for (; dev.done < n; ++dev.done) std::memcpy(dev.queue[dev.done].dst, dev.queue[dev.done].src, dev.queue[dev.done].n);
 }
 hipError_t host_malloc(void** p, size_t n, unsigned) {
-    if (dev.refuse_pinned) return hipErrorOutOfMemory;
+    if (dev.refuse_pinned && dev.nalloc >= dev.refuse_pinned - 1) return hipErrorOutOfMemory;
     *p = std::malloc(n);
     ++dev.nalloc;
     dev.live.push_back({*p, n});
     dev.pinned += (long)n;
     dev.most = std::max(dev.most, dev.pinned);
+    dev.block = std::max(dev.block, (long)n);
     return hipSuccess;
 }
 hipError_t host_free(void* p) {
@@ -100,10 +101,11 @@ extern "C" {
 
 // `reads` reads of nf fields of rows x nx floats at src through one FrameBuf,
 // converted to doubles at dst; the last one fails at its fail_copy-th copy if
-// that is not negative.  Returns the last read's error.  stats: copies of the
-// last read, pinned allocations, most pinned bytes at once, pinned bytes and
-// events left after the release, threads that converted rows in the last read
-// and threads that it was given.
+// that is not negative, and the refuse_pinned-th pinned allocation and all after
+// it are refused if that is not zero.  Returns the last read's error.  stats:
+// copies of the last read, pinned allocations, most pinned bytes at once, pinned
+// bytes and events left after the release, threads that converted rows in the
+// last read, threads that it was given, bytes of the largest pinned allocation.
 int hostcheck_frame(long rows, long nx, int nf, int reads, int late, int refuse_pinned, int fail_copy,
                     const float* src, double* dst, long* stats) {
     fake::dev = fake::Device();
@@ -137,6 +139,7 @@ int hostcheck_frame(long rows, long nx, int nf, int reads, int late, int refuse_
     stats[4] = fake::dev.nevent;
     stats[5] = (long)ids.size();
     stats[6] = (long)fb.threads;
+    stats[7] = fake::dev.block;
     return (int)e;
 }
 

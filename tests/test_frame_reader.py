@@ -21,10 +21,10 @@ def lib():
 def _read(lib, rows, nx, nf, reads=1, late=0, refuse=0, fail=-1):
     src = np.random.default_rng(rows + nx).standard_normal((nf, rows, nx)).astype(np.float32)
     dst = np.zeros((nf, rows, nx))
-    stats = (ctypes.c_long * 7)()
+    stats = (ctypes.c_long * 8)()
     err = lib.hostcheck_frame(ctypes.c_long(rows), ctypes.c_long(nx), nf, reads, late, refuse, fail,
                               src.ctypes.data_as(ctypes.c_void_p), dst.ctypes.data_as(ctypes.c_void_p), stats)
-    return err, src, dst, dict(zip(("copies", "allocs", "most", "pinned", "events", "threads", "given"),
+    return err, src, dst, dict(zip(("copies", "allocs", "most", "pinned", "events", "threads", "given", "block"),
                                      stats))
 
 
@@ -44,9 +44,10 @@ def test_every_cell_once(lib, rows, nx, nf, late):
 
 @pytest.mark.parametrize("rows, nx, nf", SHAPES)
 @pytest.mark.parametrize("late", [0, 1])
-def test_without_pinned_memory(lib, rows, nx, nf, late):
-    err, src, dst, st = _read(lib, rows, nx, nf, reads=2, late=late, refuse=1)
-    assert err == 0 and st["allocs"] == 0
+@pytest.mark.parametrize("refuse", [1, 2])        # none at all; none after the first
+def test_without_pinned_memory(lib, rows, nx, nf, late, refuse):
+    err, src, dst, st = _read(lib, rows, nx, nf, reads=2, late=late, refuse=refuse)
+    assert err == 0 and st["allocs"] < refuse and st["pinned"] == 0
     assert np.array_equal(dst, 2 * src.astype(np.float64))
 
 
@@ -67,14 +68,14 @@ def test_a_small_frame_is_one_copy_without_pinned_memory(lib, rows, nx, nf):
     assert st["copies"] == 1 and st["allocs"] == 0 and st["threads"] == 1, st
 
 
-# 42 and 7 MB: the first read; 2.4 MB: the second; 1.9 MB: the third
-@pytest.mark.parametrize("rows, nx, nf, pins_at", [(3001, 701, 5, 1), (301, 2001, 3, 1), (500, 401, 3, 2), (401, 401, 3, 3)])
-def test_pieces_are_pinned_once_4_mb_are_read(lib, rows, nx, nf, pins_at):
-    for reads in (pins_at - 1, pins_at, pins_at + 2):
-        if reads:
-            err, src, dst, st = _read(lib, rows, nx, nf, reads=reads, late=1)
-            assert err == 0 and np.array_equal(dst, reads * src.astype(np.float64))
-            assert st["allocs"] == (reads >= pins_at) and st["pinned"] == 0, st
+# 1.2 MB in two pieces; 2.4, 7 and 14 MB in three buffers; 42 MB
+@pytest.mark.parametrize("rows, nx, nf, pieces", [(500, 201, 3, 2), (500, 401, 3, 3), (301, 2001, 3, 3), (301, 4001, 3, 3),
+                                                  (3001, 701, 5, 3)])
+def test_a_piece_is_an_allocation_of_its_own(lib, rows, nx, nf, pieces):
+    err, src, dst, st = _read(lib, rows, nx, nf, reads=3, late=1)
+    assert err == 0 and np.array_equal(dst, 3 * src.astype(np.float64))
+    frame = 4 * rows * nx * nf
+    assert st["allocs"] == pieces and st["block"] <= max(1 << 20, frame // 16), st
 
 
 # rows of 14, 0.6 and 0.014 MB: a piece holds 1, 4 and 187 of them
