@@ -152,8 +152,9 @@ struct Par {
 // branch: with 1e-4 noise on the density some lane of nearly every wave takes
 // the power law in some field, and the forms evaluated field by field, each
 // behind its own branches, kept 40-52 % of the lanes idle in the radial and
-// azimuthal sweeps, which issue instructions on every cycle (384x1536x64 step
-// 4.69 -> 4.14 ms, 96x384x64 332 -> 292 us with the radial sweep's tiles).
+// azimuthal sweeps, which issue instructions on every cycle; 16 and 32 % are now
+// (384x1536x64 step 4.69 -> 4.14 ms, 96x384x64 332 -> 292 us with the radial
+// sweep's tiles).
 template <int RECON, int SIDE, int N, typename real>
 __device__ __forceinline__ void edge_means(real x, const Par<real> (&P)[N], real (&m)[N]) {
     bool any = false;
