@@ -4,12 +4,13 @@
 // Part of libpg_adjcheck.so; the product library does not contain it.
 #include <hip/hip_runtime.h>
 
-#include <atomic>
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <set>
 #include <thread>
+#include <utility>
 #include <vector>
 
 namespace fake {
