@@ -1,7 +1,7 @@
-"""Reading a 2D state back in FP32: frames of one piece, of several by one thread
-and of several by several, read often enough that the later ones go through
-pinned pieces.  Every read gives the values that were set, rounded once as a
-deviation from the background, and the same bits as the first."""
+"""Reading a 2D state back in FP32: frames of one (pageable) piece, of several
+pinned ones by one thread and of several by several.  Every read gives the values
+that were set, rounded once as a deviation from the background, and the same bits
+as the first."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 EPS = np.finfo(np.float32).eps
 
 
-# 0.15 (never pinned), 3 (at the second read), 9 and 25 MB a fluid
+# 0.15 (one piece), 3, 9 and 25 MB a fluid
 @pytest.mark.parametrize("nr, nphi", [(41, 301), (257, 1023), (600, 1300), (701, 3001)])
 @pytest.mark.parametrize("dust", [0, 1])
 def test_frame_2d_fp32(nr, nphi, dust):
